@@ -408,9 +408,9 @@ nsr_status nsr_conv1d_f32io(const float* x, const void* w, const void* bias, flo
  *                          fragment order (ceil(C_out / 128) x 4 x K x
  *                          ceil(C_in / 128) x 8192 bytes). When the
  *                          workspace also covers it (after the parts the call
- *                          needs), rows with T_out % 4 == 0 and 16-byte
- *                          aligned out / residual, and (K - 1) * dilation
- *                          <= 56, take the two-launch record path: a
+ *                          needs), rows of any length and alignment with
+ *                          K >= 7, even C_out and (K - 1) * dilation <= 56
+ *                          take the two-launch record path: a
  *                          bandwidth-bound pass writes the records (AdaIN +
  *                          Snake included in the fused entry points) and the
  *                          fragment weights, then an MFMA kernel with no

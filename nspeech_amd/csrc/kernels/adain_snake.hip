@@ -963,17 +963,23 @@ NSR_ADAIN_ROW_H(512, 22, 10)
 
 /* ------------------------------------------------ row statistics, long rows -- */
 
-/* Sum and sum of squares of one row over 1024 lanes in f64, one HBM read:
- * 16-byte loads (eight in flight per lane) when VEC4 (row 16-byte aligned,
- * T % 4 == 0), else element loads. In f64, var = S2/T - (S1/T)^2 keeps
+/* Four f32 at any 4-byte aligned address (one 16-byte access: gfx950 serves it at dword alignment). */
+typedef float nsr_float4u __attribute__((ext_vector_type(4), aligned(4)));
+NSR_DEV nsr_float4 ldf4u(const float* p) { return __builtin_nontemporal_load((const nsr_float4u*)p); }
+NSR_DEV void stf4u(float* p, nsr_float4 v) { __builtin_nontemporal_store(v, (nsr_float4u*)p); }
+
+/* Sum and sum of squares of one row (any 4-byte aligned start, any T) over
+ * 1024 lanes in f64, one HBM read with 16-byte loads, eight in flight per
+ * lane; the T % 4 last elements go to the first lanes ([512, 57601] rows:
+ * 23.8 us against 49.2 us with one element per lane and load, kernel trace). In f64, var = S2/T - (S1/T)^2 keeps
  * about 16 - log10(mean^2 / var) significant digits, far more than f32
  * output needs for any |mean| / std below 1e4. `red` holds 32 doubles. */
-template <bool VEC4, bool CACHED = false>
+template <bool CACHED = false>
 NSR_DEV void row_sums64(const float* xr, int64_t T, double* red, double& s1, double& s2) {
   NSR_NO_CONTRACT
   double a1 = 0.0, a2 = 0.0;
   const int tid = threadIdx.x;
-  if constexpr (VEC4) {
+  {
     const int64_t n4 = T >> 2;
     auto acc4 = [&](const nsr_float4* v) {
 #pragma unroll
@@ -1029,7 +1035,7 @@ NSR_DEV void row_sums64(const float* xr, int64_t T, double* red, double& s1, dou
     }
     int64_t i = (g << 12) + tid;
     for (; i < n4; i += 1024) {
-      const nsr_float4 v = ldf4(xr + 4 * i);
+      const nsr_float4 v = ldf4u(xr + 4 * i);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const double x = (double)v[e];
@@ -1037,9 +1043,8 @@ NSR_DEV void row_sums64(const float* xr, int64_t T, double* red, double& s1, dou
         a2 = __builtin_fma(x, x, a2);
       }
     }
-  } else {
-    for (int64_t i = tid; i < T; i += 1024) {
-      const double x = (double)__builtin_nontemporal_load(xr + i);
+    if (tid < (int)(T & 3)) {
+      const double x = (double)__builtin_nontemporal_load(xr + 4 * n4 + tid);
       a1 += x;
       a2 = __builtin_fma(x, x, a2);
     }
@@ -1078,12 +1083,11 @@ NSR_DEV void row_moments(double s1, double s2, int64_t T, float eps, float& mhi,
 /* Row statistics (mean, 1 / sqrt(var + eps)) of [n_rows][T] f32 into
  * a.stats: one 1024-lane workgroup per row, one read of x. Used where the
  * statistics feed another kernel (the AdaIN + Snake input of the conv). */
-template <bool VEC4>
 NSR_DEV void adain_stats(const nsr_adain_args& a) {
   __shared__ double red[32];
   const int64_t row = blockIdx.x;
   double s1, s2;
-  row_sums64<VEC4>(a.x + row * a.T, a.T, red, s1, s2);
+  row_sums64(a.x + row * a.T, a.T, red, s1, s2);
   if (threadIdx.x == 0) {
     float mhi, mlo, rstd;
     row_moments(s1, s2, a.T, a.eps, mhi, mlo, rstd);
@@ -1092,8 +1096,7 @@ NSR_DEV void adain_stats(const nsr_adain_args& a) {
   }
 }
 
-extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_stats(const nsr_adain_args a) { adain_stats<false>(a); }
-extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_stats4(const nsr_adain_args a) { adain_stats<true>(a); }
+extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_stats(const nsr_adain_args a) { adain_stats(a); }
 
 /* Rows too long to hold on chip (or unaligned rows past the resident
  * kernels' reach): a persistent grid of 1024-lane workgroups, each taking
@@ -1104,7 +1107,6 @@ extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_stats4(const nsr_a
  * row's time, so with a workgroup per CU the rows in flight (a few hundred
  * MB at most) are mostly still in the 256 MB Infinity Cache: the extra
  * traffic is mostly cache, not HBM. No scratch memory. */
-template <bool VEC4>
 NSR_DEV void adain_long(const nsr_adain_args& a, int pdt) {
   NSR_NO_CONTRACT
   __shared__ double red[32];
@@ -1118,7 +1120,7 @@ NSR_DEV void adain_long(const nsr_adain_args& a, int pdt) {
     /* the first read cached, so that the second (streamed) finds much of the row in the caches: measured on
      * MI355X at [8, 128, 131072] f32, 240.7-241.6 us against 280.0-281.0 us with both reads streamed (both
      * cached 255.0-255.5, only the second 290.9-291.9 us); the same output bits */
-    row_sums64<VEC4, true>(xr, T, red, s1, s2);
+    row_sums64<true>(xr, T, red, s1, s2);
     float mhi, mlo, rstd;
     row_moments(s1, s2, T, a.eps, mhi, mlo, rstd);
     float gam, bet, alp;
@@ -1126,22 +1128,15 @@ NSR_DEV void adain_long(const nsr_adain_args& a, int pdt) {
     const float A = (gam + 1.0f) * rstd;
     const float Bc = __builtin_fmaf(-mlo, A, bet); /* ((x - mhi) - mlo) A + beta */
     const snake_consts sc = make_snake_consts(alp);
-    if constexpr (VEC4) {
-      const int64_t n4 = T >> 2;
-      for (int64_t i = tid; i < n4; i += 1024) {
-        const nsr_float4 d = ldf4(xr + 4 * i) - mhi;
-        stf4(orow + 4 * i, adain_snake4(d, A, Bc, sc));
-      }
-    } else {
-      for (int64_t i = tid; i < T; i += 1024)
-        orow[i] = snake_eval(__builtin_fmaf(__builtin_nontemporal_load(xr + i) - mhi, A, Bc), sc);
+    const int64_t n4 = T >> 2;
+    for (int64_t i = tid; i < n4; i += 1024) {
+      const nsr_float4 d = ldf4u(xr + 4 * i) - mhi;
+      stf4u(orow + 4 * i, adain_snake4(d, A, Bc, sc));
     }
+    if (tid < (int)(T & 3)) orow[4 * n4 + tid] = snake_eval(__builtin_fmaf(xr[4 * n4 + tid] - mhi, A, Bc), sc);
   }
 }
 
 extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_long(const nsr_adain_args a, const int pdt) {
-  adain_long<false>(a, pdt);
-}
-extern "C" __global__ void __launch_bounds__(1024) nsrk_adain_long4(const nsr_adain_args a, const int pdt) {
-  adain_long<true>(a, pdt);
+  adain_long(a, pdt);
 }

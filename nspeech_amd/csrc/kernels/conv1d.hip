@@ -986,7 +986,16 @@ NSR_CONV_PC(4)
  *    tap K - 2 when it holds a record that only earlier taps read, after the
  *    last tap otherwise (then one more barrier before the next item; never
  *    for consecutive tiles of one row with an even (K - 1) dilation).
- * Two barriers per item. LDS: 256 x 528 bytes. */
+ * Two barriers per item. LDS: 256 x 528 bytes.
+ *
+ * Rows of any length: out and residual rows are accessed with 16-byte buffer
+ * operations at 4-byte alignment, whose range check works per dword (checked
+ * on gfx950: the dwords of a 16-byte load or store inside the range are
+ * served, the others read 0 or are dropped). The last quad of a row with
+ * T_out % 4 != 0 is stored dword by dword, in the row's last column tile only.
+ * At [4, 128, 57601], K = 11, the six stages of a ResBlock take 1429 us
+ * against 2839 us on the kernel for unaligned rows above (MFMA kernel, records
+ * and statistics together; 1394 us against 1319 us with T = 57600 on one box). */
 #define CV_RB 512           /* bytes per record */
 #define CV_RS 528           /* bytes per record slot in LDS */
 #define CV_RING 256         /* record slots in LDS */
@@ -1102,7 +1111,7 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
     auto calc_saddr = [&](const cv_item& im, int nt0, int jw) {
       const int quad = lane & 31, t = im.t0 + 4 * quad;
       svo = (uint32_t)(lane >> 5) * (uint32_t)a.T_out * 4u + (uint32_t)t * 4u;
-      sok = t < a.T_out ? 1u : 0u;
+      sok = (uint32_t)max(0, min(4, a.T_out - t)); /* columns of the quad inside the row */
       pin(svo);
       pin(sok);
 #pragma unroll
@@ -1124,6 +1133,7 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
     };
     auto store_staged = [&](const cv_item& im, int jw, int gap) {
       const uint32_t obytes = 4u * (uint32_t)a.C_out * (uint32_t)a.T_out;
+      const bool ragged = (a.T_out & 3) != 0 && im.t0 + CV_TW > a.T_out; /* wave-uniform */
       const nsr_rsrc orr = make_rsrc_uniform(a.out + (int64_t)im.b * a.C_out * a.T_out, obytes);
       /* the residual (variants without statistics add it here), loaded 4 passes ahead */
       const nsr_rsrc rr = make_rsrc_uniform(RESID ? a.residual + (int64_t)im.b * a.C_out * a.T_out : a.out, obytes);
@@ -1146,9 +1156,18 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
           if (p + 4 < 16) load_rq(p + 4);
         }
         /* C_out is even on this path: both rows of a pair exist or neither */
-        if (sok && im.co0 + r0 < a.C_out)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), orr, svo,
-                                                 (uint32_t)(im.co0 + r0) * (uint32_t)a.T_out * 4u, 0);
+        const uint32_t so = (uint32_t)(im.co0 + r0) * (uint32_t)a.T_out * 4u;
+        if (sok == 4u && im.co0 + r0 < a.C_out)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), orr, svo, so, 0);
+        if (ragged && im.co0 + r0 < a.C_out) {
+          /* the quad that holds the row's end (T_out % 4 columns of it), last column tile only */
+#pragma unroll
+          for (int e = 0; e < 3; ++e) {
+            const float ve = v[e]; /* a named copy: a bit_cast of the vector element itself reads element 0 */
+            if (sok < 4u && (uint32_t)e < sok)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ve), orr, svo + 4u * e, so, 0);
+          }
+        }
         for (int z = 0; z < gap; ++z) __builtin_amdgcn_s_sleep(1);
       }
     };
@@ -1262,7 +1281,8 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
     nsr_float4 rv[RESID ? 2 : 1][RESID ? 2 : 1][RESID ? 4 : 1];
     auto load_resid = [&](const cv_item& it, int tb) {
       const nsr_rsrc rr = make_rsrc_uniform(a.residual + (int64_t)it.b * a.C_out * a.T_out, obytes);
-      const uint32_t tc = (uint32_t)min(it.t0 + wt * 64 + tb * 32 + 4 * (l32 >> 2), a.T_out - 4);
+      /* columns past T_out read the next row or, past the buffer, 0 (the range check is per dword): unused */
+      const uint32_t tc = (uint32_t)(it.t0 + wt * 64 + tb * 32 + 4 * (l32 >> 2));
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll

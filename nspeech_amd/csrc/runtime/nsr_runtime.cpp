@@ -788,9 +788,7 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
   }
   // Rows past the on-chip budget: statistics over one read, then a second read to apply (persistent grid,
   // one 1024-lane workgroup per CU, no scratch).
-  const bool rows16 = T % 4 == 0 && aligned(x, 16) && aligned(out, 16);
-  return launch(rows16 ? K_nsrk_adain_long4 : K_nsrk_adain_long, (unsigned)std::min<int64_t>(n_rows, dm->n_cu), 1,
-                1024, 0, stream, params);
+  return launch(K_nsrk_adain_long, (unsigned)std::min<int64_t>(n_rows, dm->n_cu), 1, 1024, 0, stream, params);
 }
 
 nsr_status nsr_adain_snake_f16(const void* x, const void* gamma, const void* beta, const void* alpha,
@@ -1501,11 +1499,10 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   if (st != NSR_OK) return st;
   const int64_t D = (int64_t)(a.K - 1) * a.dilation;
   const int64_t TLe = kCvTW + D + (D & 1);
-  const bool rows16 = a.T_out % 4 == 0 && aligned(a.out, 16) && (!a.residual || aligned(a.residual, 16));
   // TLe <= 184 leaves 72 ring slots outside a window, which with the 56 rows after the ring stage a 128-row tile.
   // Below K = 7 the records pass (x read, records written) costs more than the one-launch kernels lose to
   // their per-element work (measured on MI355X at [8, 128, 115200]: K = 3 about 540 us against 370 us).
-  if (!records || a.K < 7 || !rows16 || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0)
+  if (!records || a.K < 7 || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0)
     return conv_launch(fused, a, stream, what, emitted);
   const int64_t Tp = (int64_t)a.T_in + 2 * a.padding;
   const int64_t n_ch = (a.C_in + 127) / 128, n_co = (a.C_out + 127) / 128;
@@ -1519,7 +1516,6 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   void* pp[] = {&a, &xs, &wf};
   st = launch(fused ? K_nsrk_conv_presplit_adain_snake : K_nsrk_conv_presplit, (unsigned)blocks, 1, 256, 0, stream, pp);
   if (st != NSR_OK) return st;
-  a.pad_ = 1;
   const int64_t tiles = (int64_t)cdiv_u(a.T_out, kCvTW) * n_co * a.B;
   if (tiles > 0x7fffffffLL) return fail(NSR_ERR_UNSUPPORTED, "%s: too many tiles", what);
   const bool stats = a.row_part != nullptr;
@@ -1567,8 +1563,7 @@ static nsr_status conv_launch_stats(bool fused, nsr_conv_args& a, float eps, flo
     s.eps = eps;
     s.inv_t = 1.0f / (float)a.T_out;
     void* ps[] = {&s};
-    const bool rows16 = a.T_out % 4 == 0 && aligned(a.out, 16);
-    st = launch(rows16 ? K_nsrk_adain_stats4 : K_nsrk_adain_stats, (unsigned)rows, 1, 1024, 0, stream, ps);
+    st = launch(K_nsrk_adain_stats, (unsigned)rows, 1, 1024, 0, stream, ps);
   }
   a.row_part = nullptr;
   return st;
@@ -1702,8 +1697,7 @@ static nsr_status adain_conv_impl(const float* x, const float* x_stats, const vo
     s.eps = eps;
     s.inv_t = 1.0f / (float)T;
     void* p1[] = {&s};
-    const bool rows16 = T % 4 == 0 && aligned(x, 16);
-    st = launch(rows16 ? K_nsrk_adain_stats4 : K_nsrk_adain_stats, (unsigned)(B * C_in), 1, 1024, 0, stream, p1);
+    st = launch(K_nsrk_adain_stats, (unsigned)(B * C_in), 1, 1024, 0, stream, p1);
   }
   if (st == NSR_OK) {
     nsr_conv_args a;

@@ -1,0 +1,120 @@
+"""Conv rows that do not start on 16 bytes (T % 4 != 0, as the generator's last
+stage gives with its reflection pad): the record kernels and the row statistics
+on every remainder of T mod 4, at tile edges and ends.
+
+The float64 conv of the float64 AdaIN + Snake is the reference. The bar is the
+f32 accumulation bound: n = C_in K products, each with the input's own error of
+at most 2e-6 |y|, summed in some order with n u relative to sum |w y| (u =
+2^-24): (2e-6 + n u) sum |w y| + 2 u |out|. The output and the residual sit in
+buffers with sentinels around them."""
+import numpy as np
+import pytest
+import torch
+
+from nspeech_amd import abi, configs
+
+from ._util import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(x, gam, bet, alp, w, bias, res, pad, dil):
+    """float64 output and sum |w y| of the fused stage."""
+    x = x.double()
+    m = x.mean(-1, keepdim=True)
+    y = (x - m) / torch.sqrt((x - m).square().mean(-1, keepdim=True) + 1e-5)
+    y = y * (1.0 + gam.double()[:, :, None]) + bet.double()[:, :, None]
+    al = alp.double()[None, :, None]
+    y = y + torch.sin(al * y).square() / (al + 1e-9)
+    T, K = x.shape[-1], w.shape[2]
+    yp = torch.nn.functional.pad(y, (pad, pad))
+    out = bias.double()[None, :, None].expand(x.shape[0], -1, T).clone()
+    mag = torch.zeros_like(out)
+    for k in range(K):
+        s = yp[:, :, k * dil:k * dil + T].contiguous()
+        for b in range(x.shape[0]):
+            out[b] += w[:, :, k].double().contiguous() @ s[b]
+            mag[b] += w[:, :, k].double().abs().contiguous() @ s[b].abs()
+    if res is not None:
+        out, mag = out + res.double(), mag + res.double().abs()
+    return out, mag
+
+
+@pytest.mark.parametrize("B,C_in,C_out,T,K,dil,res", [
+    (1, 128, 128, 1, 7, 1, True),       # one column
+    (2, 128, 128, 3, 11, 5, False),     # shorter than a quad
+    (1, 128, 128, 129, 7, 1, True),     # one column past a 128-column tile
+    (2, 128, 128, 130, 7, 3, True),
+    (1, 128, 128, 127, 11, 5, True),    # one column short of a tile
+    (2, 256, 256, 255, 7, 1, False),    # two channel chunks and blocks
+    (1, 144, 200, 601, 9, 5, True),     # partial channel chunk and block
+    (3, 64, 96, 1001, 8, 1, True),      # odd (K - 1) dilation
+    (1, 128, 128, 19201, 11, 5, True),  # many tiles per workgroup are not reached; tiles past one per CU are below
+    (2, 128, 128, 19203, 7, 5, True),
+    (1, 64, 64, 601, 5, 2, True),       # K < 7: the one-launch kernels
+    (2, 128, 128, 1003, 3, 5, True),
+    (1, 128, 128, 19201, 3, 1, False),
+    (1, 256, 128, 333, 5, 3, True),
+])
+def test_fused_stage_ragged_rows(B, C_in, C_out, T, K, dil, res):
+    say("conv ragged rows", B, C_in, C_out, T, K, dil, res)
+    g = configs.rng(B * 7 + C_in + 3 * K + dil + T)
+    t = lambda a, dt=np.float32: torch.from_numpy(np.ascontiguousarray(a.astype(dt))).cuda()  # noqa: E731
+    x = t(g.standard_normal((B, C_in, T)) * 1.3 + 0.2)
+    w = t(g.standard_normal((C_out, C_in, K)) * 0.05, np.float16)
+    bias = t(g.standard_normal(C_out), np.float16)
+    gam, bet, alp = t(g.standard_normal((B, C_in)) * 0.1), t(g.standard_normal((B, C_in)) * 0.1), t(g.uniform(0.5, 1.5, C_in))
+    r = t(g.standard_normal((B, C_out, T))) if res else None
+    pad = (K - 1) * dil // 2
+    if 2 * pad != (K - 1) * dil:
+        pad = None
+    wp = abi.conv1d_pack_f16(w)
+    n = B * C_out * T
+    if pad is None:  # T_out != T: compare the two paths' plain conv instead of a reference of equal length
+        pad = (K - 1) * dil // 2
+        T_out = T + 2 * pad - dil * (K - 1)
+        r = t(g.standard_normal((B, C_out, T_out))) if res else None
+        o1, s1 = abi.conv1d_f16w_packed_stats(x, wp, bias, r, padding=pad, dilation=dil, records=True)
+        o0 = abi.conv1d_f16w_packed(x, wp, bias, r, padding=pad, dilation=dil)
+        assert torch.equal(o1, o0)
+        return
+    ref, mag = _reference(x, gam, bet, alp, w, bias, r, pad, dil)
+    bar = (2e-6 + C_in * K * 2.0 ** -24) * mag + 2.0 ** -23 * ref.abs()
+    outs = []
+    for records in (True, False):
+        for stats in (True, False):
+            buf = torch.full((n + 32,), -7.0, device="cuda")
+            out = buf[16:16 + n].view(B, C_out, T)
+            o, st = abi.adain_snake_conv1d_chain(x, gam, bet, alp, wp, bias, r, want_stats=stats, padding=pad, dilation=dil,
+                                                 out=out, records=records)
+            assert bool((buf[:16] == -7.0).all()) and bool((buf[16 + n:] == -7.0).all()), "wrote outside the output"
+            worst = float(((o.double() - ref).abs() / bar).max())
+            assert worst <= 1.0, f"records={records} stats={stats}: {worst:.2f} of the bar"
+            outs.append(o)
+            if stats:
+                d = o.double()
+                mean, var = d.mean(-1), d.var(-1, unbiased=False)
+                st = st.double().view(B, C_out, 2)
+                spread = torch.sqrt(var + 1e-5)
+                assert bool(((st[:, :, 0] - mean).abs() <= 1e-5 * torch.maximum(mean.abs(), spread)).all())
+                assert bool(((st[:, :, 1] * spread - 1.0).abs() <= 1e-5).all())
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0]), "paths differ"
+
+
+def test_ragged_rows_from_misaligned_views():
+    """Input, residual and output 4 bytes past a 16-byte boundary, T a multiple of 4 and not."""
+    for T in (512, 517):
+        g = configs.rng(T)
+        B, C, K, dil, pad = 2, 128, 7, 1, 3
+        n = B * C * T
+        flat = lambda: torch.from_numpy(g.standard_normal(n + 8).astype(np.float32)).cuda()  # noqa: E731
+        xb, rb, ob = flat(), flat(), flat()
+        x, r, out = (v[1:1 + n].view(B, C, T) for v in (xb, rb, ob))
+        w = torch.from_numpy((g.standard_normal((C, C, K)) * 0.05).astype(np.float16)).cuda()
+        wp = abi.conv1d_pack_f16(w)
+        want, _ = abi.conv1d_f16w_packed_stats(x.clone(), wp, None, r.clone(), padding=pad, dilation=dil)
+        keep = ob.clone()
+        got, _ = abi.conv1d_f16w_packed_stats(x, wp, None, r, padding=pad, dilation=dil, out=out)
+        assert torch.equal(got, want)
+        assert torch.equal(ob[:1], keep[:1]) and torch.equal(ob[1 + n:], keep[1 + n:])
