@@ -341,24 +341,24 @@ NSR_DEV float sum_lanes8(float v) {
  * of the block lie before T_out, so no column is masked; the arithmetic is
  * the same either way (a masked column adds 0 to the sum and fma(0, 0, .)
  * to M2), so a block's statistics do not depend on the variant. */
-template <bool FULLB>
-NSR_DEV void emit_rows8_v(const nsr_float4 (&ov)[2][4], int t, int tb, int T_out, int l32, int co_lane, int C_out,
+template <bool FULLB, int MT = 2>
+NSR_DEV void emit_rows8_v(const nsr_float4 (&ov)[MT][4], int t, int tb, int T_out, int l32, int co_lane, int C_out,
                           int64_t row0, int nblk, int blk, float* part) {
   const int nv = FULLB ? 4 : max(0, min(4, T_out - t));
   const float n = FULLB ? 32.f : (float)max(0, min(32, T_out - tb)); /* valid columns of the block */
   const float inv_n = FULLB ? 1.0f / 32.0f : 1.0f / fmaxf(n, 1.f);
-  float mean[8], m2[8];
+  float mean[4 * MT], m2[4 * MT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 4 * MT; ++i) {
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) s += (FULLB || e < nv) ? ov[i >> 2][i & 3][e] : 0.f;
     mean[i] = s;
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) mean[i] = sum_lanes8(mean[i]) * inv_n;
+  for (int i = 0; i < 4 * MT; ++i) mean[i] = sum_lanes8(mean[i]) * inv_n;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 4 * MT; ++i) {
     float qv = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -368,22 +368,23 @@ NSR_DEV void emit_rows8_v(const nsr_float4 (&ov)[2][4], int t, int tb, int T_out
     m2[i] = qv;
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) m2[i] = sum_lanes8(m2[i]);
+  for (int i = 0; i < 4 * MT; ++i) m2[i] = sum_lanes8(m2[i]);
   if (l32 < 4 && (FULLB || n > 0.f)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < 4 * MT; ++i) {
       const int co = co_lane + 32 * (i >> 2) + 8 * (i & 3);
       if (co < C_out) *(nsr_float2*)(part + 2 * ((row0 + co) * nblk + blk)) = nsr_float2{mean[i], m2[i]};
     }
   }
 }
 
-NSR_DEV void emit_rows8(const nsr_float4 (&ov)[2][4], int t, int tb, int T_out, int l32, int co_lane, int C_out,
+template <int MT>
+NSR_DEV void emit_rows8(const nsr_float4 (&ov)[MT][4], int t, int tb, int T_out, int l32, int co_lane, int C_out,
                         int64_t row0, int nblk, int blk, float* part) {
   if (tb + 32 <= T_out) /* wave-uniform */
-    emit_rows8_v<true>(ov, t, tb, T_out, l32, co_lane, C_out, row0, nblk, blk, part);
+    emit_rows8_v<true, MT>(ov, t, tb, T_out, l32, co_lane, C_out, row0, nblk, blk, part);
   else
-    emit_rows8_v<false>(ov, t, tb, T_out, l32, co_lane, C_out, row0, nblk, blk, part);
+    emit_rows8_v<false, MT>(ov, t, tb, T_out, l32, co_lane, C_out, row0, nblk, blk, part);
 }
 
 template <bool FUSED, bool RESID, int NU, bool STATS = false>
@@ -1495,6 +1496,205 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
 NSR_CONV_PR1(nsrk_conv1d_pr_f16x2, false)
 NSR_CONV_PR1(nsrk_conv1d_pr_res_f16x2, true)
 
+/* ------------------------------------- conv on records, small output tiles -- */
+
+/* The record kernel for outputs with too few 128 x 128 tiles to fill the chip: one 256-lane workgroup per
+ * tile of 64 MT channels x 64 columns, 2 x 2 waves of 32 MT channels x 32 columns, several workgroups per CU
+ * where LDS and registers allow. A workgroup copies its window of 64 + (K - 1) dilation records of one
+ * channel chunk straight to LDS (buffer_load ... lds) and then only multiplies:
+ * B fragments from LDS, A fragments from the fragment weights into two register sets, each reloaded for
+ * the tap after next as its steps are issued. Records r and r + P (P = 48 or 64, a multiple of 16) share
+ * one 1040-byte slot, so that one 64-lane load of 16 bytes fills a slot and 16 lanes reading one chunk of
+ * consecutive records hit 16 bank groups. Products are added in the order of the other conv kernels
+ * (chunk, tap, 16-channel step, hi then lo): the same bits. That order makes each accumulator one chain of
+ * dependent MFMAs, about 66 cycles apart at MT = 1 (32 issue cycles each) and 47 at MT = 2: with one wave per
+ * SIMD this chain bounds the kernel. GPU time of ResBlocks (graph replays, against the 128 x 128 tiles):
+ * [1, 256, 3200] K = 11 181 us (MT = 1; MT = 2 196) against 282; [1, 128, 9601] K = 11, two dilations, 102 us
+ * (MT = 2; MT = 1 111) against 138; [7, 256, 2460] K = 11, two dilations, 322 us against 386. Tried and not
+ * faster: every chunk's window staged at once, the weights read ahead into the XCD's L2, B fragments read
+ * three steps ahead. */
+#define CV_PS 1040
+template <int MT, bool RESID, bool STATS>
+NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8_t* wf) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t cv_ps[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wco = wave >> 1, wt = wave & 1;
+  const int hl = lane >> 5, l32 = lane & 31, c4 = lane & 3;
+  const int D = (a.K - 1) * a.dilation, W = CV_TT + D, Tp = a.T_out + D;
+  const int P = W <= 96 ? 48 : 64;
+  const int n_t = (a.T_out + CV_TT - 1) / CV_TT, n_ch = (a.C_in + CV_CI - 1) / CV_CI;
+
+  /* tiles with the channel block slowest, an eighth of them per XCD: an XCD's L2 then holds one block's weights */
+  const int tile = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
+  const int tb_all = n_t * a.B, cb = tile / tb_all, rt = tile - cb * tb_all;
+  const int b = rt / n_t, t0 = (rt - b * n_t) * CV_TT, co0 = cb * 64 * MT;
+  const int cow = co0 + 32 * MT * wco;               /* the wave's first channel */
+  const int t = t0 + 32 * wt + 4 * (l32 >> 2);       /* this lane's column quad after the quad transpose */
+
+  const uint32_t obytes = 4u * (uint32_t)a.C_out * (uint32_t)a.T_out;
+  uint32_t braw[MT][4];
+  nsr_float4 rv[RESID ? MT : 1][RESID ? 4 : 1];
+  {
+    const uint16_t* bsrc = a.bias ? a.bias : (const uint16_t*)a.w; /* any readable halves when there is no bias */
+    const nsr_rsrc rr = make_rsrc_uniform(RESID ? a.residual + (int64_t)b * a.C_out * a.T_out : a.out, obytes);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int co = cow + 32 * m + 8 * q + 4 * hl + c4;
+        braw[m][q] = bsrc[min(co, a.C_out - 1)];
+        /* columns past T_out: the next row's, or 0 past the buffer; unused */
+        if constexpr (RESID)
+          rv[m][q] = __builtin_bit_cast(nsr_float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        rr, ((uint32_t)co * (uint32_t)a.T_out + (uint32_t)t) * 4u, 0, 0));
+      }
+  }
+
+  /* A fragments: step s = (chunk, tap) of the reduction, two sets */
+  const uint32_t kstride = (uint32_t)n_ch * 8192u, cbstride = (uint32_t)a.K * kstride;
+  const int n_cb32 = ((a.C_out + CV_CO - 1) / CV_CO) * 4;
+  const nsr_rsrc wr = make_rsrc_uniform(wf, (uint32_t)n_cb32 * cbstride);
+  const uint32_t wvo = (uint32_t)lane * 16u, wbase = (uint32_t)(cow / 32) * cbstride;
+  nsr_h8 A0[MT][8], A1[MT][8];
+  auto a_off = [&](int ch, int k) { return wbase + (uint32_t)k * kstride + (uint32_t)ch * 8192u; };
+  auto load_a = [&](nsr_h8 (&A)[MT][8], uint32_t off) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        A[m][g] = __builtin_bit_cast(nsr_h8, __builtin_amdgcn_raw_buffer_load_b128(wr, wvo, off + m * cbstride + g * 1024u, 0));
+  };
+
+  nsr_f32x16 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[m][i] = 0.f;
+
+  const uint32_t rvo = (uint32_t)hl * (uint32_t)P * CV_RB + (uint32_t)l32 * 16u;
+  int ch2 = 0, k2 = 0; /* the tap whose fragments are loaded next */
+  auto next2 = [&]() {
+    const uint32_t off = a_off(ch2, k2);
+    if (++k2 == a.K) {
+      k2 = 0;
+      if (ch2 + 1 < n_ch) ++ch2; /* past the last tap: reloads of the last chunk's first taps, unused */
+    }
+    return off;
+  };
+  load_a(A0, next2());
+  load_a(A1, next2());
+
+  int s = 0; /* taps done, over all chunks */
+  for (int ch = 0; ch < n_ch; ++ch) {
+    if (ch > 0) __syncthreads(); /* every wave is done with the previous chunk's records */
+    const nsr_rsrc xr = make_rsrc_uniform(xs + ((int64_t)b * n_ch + ch) * Tp * CV_RB, (uint32_t)Tp * (uint32_t)CV_RB);
+    for (int p = wave; p < P; p += 4) {
+      /* records t0 + p (lanes 0-31) and t0 + p + P; those past the window are not read, and past the last
+       * record of the row the load is dropped: such columns lie past T_out */
+      if (hl == 0 || p + P < W)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(cv_ps + (uint32_t)p * CV_PS), 16, rvo,
+                                                 (uint32_t)(t0 + p) * CV_RB, 0, 0);
+    }
+    NSR_WAIT_VMCNT(0);
+    __syncthreads();
+    int k = 0;
+    auto step = [&](nsr_h8 (&A)[MT][8]) {
+      const int j = 32 * wt + l32 + k * a.dilation;
+      const uint32_t va = (uint32_t)j * CV_PS - (j >= P ? (uint32_t)P * CV_PS - CV_RB : 0u) + (uint32_t)hl * 16u;
+      const uint32_t off = next2();
+      nsr_h8 Bh[2], Bl[2];
+      auto ld = [&](int buf, int g) {
+        Bh[buf] = *(const nsr_h8*)(cv_ps + va + 32 * g);
+        Bl[buf] = *(const nsr_h8*)(cv_ps + va + 256 + 32 * g);
+      };
+      ld(0, 0);
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const int cur = g & 1;
+        if (g + 1 < 8) ld(cur ^ 1, g + 1);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[m][g], Bh[cur], acc[m], 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[m][g], Bl[cur], acc[m], 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          A[m][g] = __builtin_bit_cast(nsr_h8, __builtin_amdgcn_raw_buffer_load_b128(wr, wvo, off + m * cbstride + g * 1024u, 0));
+      }
+      /* order: step g + 1's reads, step g's MFMAs, its reloads */
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+      for (int g = 0; g < 7; ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * MT, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, MT, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * MT, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, MT, 0);
+      ++s;
+      ++k;
+    };
+    /* the register sets alternate over all taps: with an odd K a chunk may start on either */
+    if (s & 1) step(A1);
+    while (k + 1 < a.K) {
+      step(A0);
+      step(A1);
+    }
+    if (k < a.K) step(A0);
+  }
+  NSR_WAIT_VMCNT(0); /* the last reloads, unused */
+
+  const nsr_rsrc orr = make_rsrc_uniform(a.out + (int64_t)b * a.C_out * a.T_out, obytes);
+  const bool ragged = (a.T_out & 3) != 0 && t0 + CV_TT > a.T_out; /* workgroup-uniform */
+  const int nq = a.T_out - t;                                     /* columns of the row from t on */
+  nsr_float4 ov[MT][4];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4] = {acc[m][4 * q], acc[m][4 * q + 1], acc[m][4 * q + 2], acc[m][4 * q + 3]};
+      float x1[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x1[r] = quad_xor1(v[r ^ 1]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = ((r ^ c4) & 1) ? x1[r] : v[r];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x1[r] = quad_xor2(v[r ^ 2]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = ((r ^ c4) & 2) ? x1[r] : v[r];
+      const float bv = a.bias ? f16_bits_to_f32((uint16_t)braw[m][q]) : 0.f;
+      nsr_float4 o = {v[0] + bv, v[1] + bv, v[2] + bv, v[3] + bv};
+      if constexpr (RESID) o += rv[m][q];
+      ov[m][q] = o;
+      const uint32_t co = (uint32_t)(cow + 32 * m + 8 * q + 4 * hl + c4);
+      const uint32_t oo = (co * (uint32_t)a.T_out + (uint32_t)t) * 4u;
+      if (nq >= 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, o), orr, oo, 0, 0);
+      if (ragged) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const float oe = o[e];
+          if (nq < 4 && e < nq) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, oe), orr, oo + 4u * e, 0, 0);
+        }
+      }
+    }
+  if constexpr (STATS)
+    emit_rows8(ov, t, t0 + 32 * wt, a.T_out, l32, cow + 4 * hl + c4, a.C_out, (int64_t)b * a.C_out, (a.T_out + 31) >> 5,
+               (t0 + 32 * wt) >> 5, a.row_part);
+}
+
+#define NSR_CONV_PS1(NAME, MT, RESID)                                                                \
+  extern "C" __global__ void __launch_bounds__(256, 2)                                              \
+      NAME(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {           \
+    conv_ps_body<MT, RESID, false>(a, xs, wf);                                                \
+  }                                                                                                 \
+  extern "C" __global__ void __launch_bounds__(256, 2)                                              \
+      NAME##_st(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {      \
+    conv_ps_body<MT, RESID, true>(a, xs, wf);                                                 \
+  }
+NSR_CONV_PS1(nsrk_conv1d_ps1_f16x2, 1, false)
+NSR_CONV_PS1(nsrk_conv1d_ps1_res_f16x2, 1, true)
+NSR_CONV_PS1(nsrk_conv1d_ps2_f16x2, 2, false)
+NSR_CONV_PS1(nsrk_conv1d_ps2_res_f16x2, 2, true)
+
 /* Records and fragment weights for nsrk_conv1d_pr*. Record tp (tp = 0 ..
  * T_in + 2 padding - 1, input column tp - padding) of channel chunk ch holds
  * y = x (or snake(AdaIN(x)) in the fused form, with the row statistics in
@@ -1541,18 +1741,10 @@ NSR_DEV void conv_presplit(const nsr_conv_args& a, uint8_t* xs, uint8_t* wf) {
     const int k = (int)(grp % a.K);
     const int cb = (int)(grp / a.K);
     const int co = 32 * cb + (ln & 31), ci0 = CV_CI * ch + 16 * g + 8 * (ln >> 5);
-    uint32_t hv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint32_t lo16 = 0, hi16 = 0;
-      if (co < a.C_out) {
-        const uint16_t* wrow = a.w + ((int64_t)co * a.K + k) * a.C_in;
-        if (ci0 + 2 * e < a.C_in) lo16 = wrow[ci0 + 2 * e];
-        if (ci0 + 2 * e + 1 < a.C_in) hi16 = wrow[ci0 + 2 * e + 1];
-      }
-      hv[e] = lo16 | (hi16 << 16);
-    }
-    *(nsr_uint4*)(wf + f * 16) = nsr_uint4{hv[0], hv[1], hv[2], hv[3]};
+    /* 8 channels: C_in is a multiple of 16 and the packed weights 16-byte aligned */
+    nsr_uint4 v = {0u, 0u, 0u, 0u};
+    if (co < a.C_out && ci0 < a.C_in) v = *(const nsr_uint4*)(a.w + ((int64_t)co * a.K + k) * a.C_in + ci0);
+    *(nsr_uint4*)(wf + f * 16) = v;
     return;
   }
   const int bc = lb / nblk; /* b * n_ch + ch */

@@ -1524,9 +1524,25 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   static const KId ids[2][3] = {{K_nsrk_conv1d_pr_f16x2, K_nsrk_conv1d_pr_f16x2_st, K_nsrk_conv1d_pr_f16x2_st32},
                                 {K_nsrk_conv1d_pr_res_f16x2, K_nsrk_conv1d_pr_res_f16x2_st,
                                  K_nsrk_conv1d_pr_res_f16x2_st32}};
-  // one workgroup per CU, a multiple of 8 (the kernel's XCD split) when there are enough tiles
-  int64_t grid = std::min<int64_t>(tiles, dm->n_cu);
-  if (grid >= 8) grid = grid / 8 * 8;
+  // 128 x 128 tiles run one per CU: when the last of at most two rounds leaves 30% of the chip idle, the kernel
+  // of 64 MT x 64 tiles is faster. Measured (MI355X, us per ResBlock, graph replays; 128 x 128 / MT = 1 / MT = 2):
+  // 14 tiles 184 / 115 / 125, 50 282 / 181 / 196, 76 138 / 111 / 102, 100 161 / 132 / 126, 151 193 / 191 / 195,
+  // 200 187 / 206 / 191, 226 149 / 151 / 145, 280 386 / 322 / 338, 302 241 / 211 / 219, 452 286 / 300 / 298.
+  // MT = 1 (four times the tiles) while they fit one per CU, and past one round of the large tiles.
+  const int64_t rounds = (tiles + dm->n_cu - 1) / dm->n_cu;
+  if (rounds <= 2 && 10 * tiles <= 7 * rounds * dm->n_cu) {
+    static const KId ps[2][2][2] = {{{K_nsrk_conv1d_ps1_f16x2, K_nsrk_conv1d_ps1_f16x2_st},
+                                     {K_nsrk_conv1d_ps1_res_f16x2, K_nsrk_conv1d_ps1_res_f16x2_st}},
+                                    {{K_nsrk_conv1d_ps2_f16x2, K_nsrk_conv1d_ps2_f16x2_st},
+                                     {K_nsrk_conv1d_ps2_res_f16x2, K_nsrk_conv1d_ps2_res_f16x2_st}}};
+    const int mt = 4 * tiles <= dm->n_cu || rounds == 2 ? 1 : 2;
+    const unsigned slots = D <= 32 ? 48 : 64;  // record slots in LDS: 64 + D <= 2 * slots
+    const int64_t grid = (int64_t)cdiv_u(a.T_out, 64) * cdiv_u(a.C_out, 64 * mt) * a.B;
+    return launch(ps[mt - 1][a.residual != nullptr][stats], (unsigned)grid, 1, 256, slots * 1040, stream, pp);
+  }
+  // one workgroup per CU, a multiple of 8 (the kernel's XCD split), never fewer than there are tiles below that:
+  // rounded down, 151 tiles gave some of 144 workgroups a second tile (256 against 193 us per ResBlock)
+  const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((tiles + 7) / 8 * 8, dm->n_cu >= 8 ? dm->n_cu / 8 * 8 : dm->n_cu));
   const int kv = stats ? (a.T_out % 32 == 0 ? 2 : 1) : 0;
   return launch(ids[a.residual != nullptr][kv], (unsigned)grid, 1, 512, kCvRingLds, stream, pp);
 }
