@@ -376,9 +376,7 @@ nsr_status nsr_attention_decode_f16(const void* q, const void* k, const void* v,
  * dilation <= 64; T_in, T_out < 2^23; stride != 1 returns
  * NSR_ERR_UNSUPPORTED, and so do shapes whose rows of one batch reach
  * 4 GiB (4 C_in T_in or 4 C_out T_out >= 2^32: one buffer descriptor
- * addresses a batch's rows). The same holds for every conv entry point. Rows that start 16-byte aligned (T_in % 4 == 0,
- * T_out % 4 == 0, 16-byte aligned x / out / residual) take the faster
- * producer/consumer kernels. Packs the weights into the caller's workspace
+ * addresses a batch's rows). The same holds for every conv entry point. Packs the weights into the caller's workspace
  * (NSR_WS_PACKED_WEIGHTS, see nsr_conv1d_workspace_bytes) on every call and
  * allocates nothing; callers that convolve repeatedly with the same weights
  * pack once with nsr_conv1d_pack_f16 and call nsr_conv1d_f16w_packed.
@@ -409,7 +407,8 @@ nsr_status nsr_conv1d_f32io(const float* x, const void* w, const void* bias, flo
  *                          ceil(C_in / 128) x 8192 bytes). When the
  *                          workspace also covers it (after the parts the call
  *                          needs), rows of any length and alignment with
- *                          K >= 7, even C_out and (K - 1) * dilation <= 56
+ *                          K >= 7 (K >= 3 when C_in or C_out is above 128),
+ *                          even C_out and (K - 1) * dilation <= 56
  *                          take the two-launch record path: a
  *                          bandwidth-bound pass writes the records (AdaIN +
  *                          Snake included in the fused entry points) and the

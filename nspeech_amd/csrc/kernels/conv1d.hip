@@ -108,6 +108,20 @@ NSR_DEV cv_coef cv_row_coef(const nsr_conv_args& a, int b, int ci) {
 }
 
 
+/* Columns t .. t + 3 of an output row at byte offset `off`, `n` of them inside the row (n <= 0: none). A quad
+ * that the row's end cuts (rows with T_out % 4 != 0) is stored column by column; `ragged` (wave-uniform) says
+ * that the tile may hold one. */
+NSR_DEV void store_quad(nsr_rsrc r, uint32_t off, nsr_float4 v, int n, bool ragged) {
+  if (n >= 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), r, off, 0, 0);
+  if (ragged) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const float ve = v[e]; /* a named copy: a bit_cast of the vector element itself reads element 0 */
+      if (n < 4 && e < n) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ve), r, off + 4u * e, 0, 0);
+    }
+  }
+}
+
 template <bool FUSED, int NP>
 NSR_DEV void conv_body(const nsr_conv_args& a) {
   extern __shared__ uint16_t cv_lds[];
@@ -296,8 +310,8 @@ NSR_DEV void conv_body(const nsr_conv_args& a) {
 
 /*
  * Resident-weight variant for C_in <= 128, C_out <= 128 and K <= 3 (the
- * resblock's kernel-size-3 convs) with 16-byte aligned rows (T_in % 4 ==
- * T_out % 4 == 0). The whole packed weight tensor, [K][128 co][128 ci] f16
+ * resblock's kernel-size-3 convs), rows of any length (16-byte buffer
+ * accesses at 4-byte alignment, range-checked per dword). The whole packed weight tensor, [K][128 co][128 ci] f16
  * zero-padded, is loaded into LDS once per workgroup and stays there
  * (<= 102 KB), next to one staged input tile. One 512-lane workgroup per
  * CU, persistent over the tiles, in two roles that overlap:
@@ -550,7 +564,7 @@ NSR_DEV void conv_rw_body(const nsr_conv_args& a) {
       nsr_float4 rv[RESID ? 2 : 1][RESID ? 4 : 1];
       if constexpr (RESID) {
         const nsr_rsrc rr = make_rsrc_uniform(a.residual + (int64_t)b * a.C_out * a.T_out, obytes);
-        const uint32_t tc = (uint32_t)min(t, a.T_out - 4);
+        const uint32_t tc = (uint32_t)t; /* columns past T_out: the next row's, or 0 past the buffer; unused */
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -608,6 +622,7 @@ NSR_DEV void conv_rw_body(const nsr_conv_args& a) {
       __syncthreads(); /* done with this tile's input */
       if (n < cnt) {
         const nsr_rsrc orr = make_rsrc_uniform(a.out + (int64_t)b * a.C_out * a.T_out, obytes);
+        const bool ragged = (a.T_out & 3) != 0 && t0 + CV_TT > a.T_out; /* wave-uniform */
         nsr_float4 ov[STATS ? 2 : 1][STATS ? 4 : 1];
 #pragma unroll
         for (int m = 0; m < 2; ++m)
@@ -628,9 +643,7 @@ NSR_DEV void conv_rw_body(const nsr_conv_args& a) {
             const uint32_t co = (uint32_t)(wco * 64 + m * 32 + 8 * q + 4 * hl + c4);
             nsr_float4 o = {v[0] + bias[m][q], v[1] + bias[m][q], v[2] + bias[m][q], v[3] + bias[m][q]};
             if constexpr (RESID) o += rv[m][q];
-            if (t < a.T_out) /* T_out % 4 == 0: t < T_out covers t + 3 */
-              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, o), orr,
-                                                     (co * (uint32_t)a.T_out + (uint32_t)t) * 4u, 0, 0);
+            store_quad(orr, (co * (uint32_t)a.T_out + (uint32_t)t) * 4u, o, a.T_out - t, ragged);
             if constexpr (STATS) ov[m][q] = o;
           }
         if constexpr (STATS)
@@ -662,7 +675,7 @@ NSR_CONV_RW(4)
 
 /*
  * Streamed-weight producer/consumer variant: any K, C_in in chunks of 128,
- * C_out in blocks of 128, 16-byte aligned rows (T_in % 4 == T_out % 4 == 0)
+ * C_out in blocks of 128, rows of any length
  * and a staged window (TL + 3 alignment columns) of at most 128 columns.
  * One 512-lane workgroup per CU, persistent over the items (tile, input
  * chunk), tiles ordered channel block fastest:
@@ -849,7 +862,7 @@ NSR_DEV void conv_pc_body(const nsr_conv_args& a) {
           /* at the tile's last tap, ahead of the weight load, so the epilogue waits for it alone */
           if (k == a.K - 1 && last_chunk) {
             const nsr_rsrc rr = make_rsrc_uniform(a.residual + (int64_t)b * a.C_out * a.T_out, obytes);
-            const uint32_t tc = (uint32_t)min(t, a.T_out - 4);
+            const uint32_t tc = (uint32_t)t; /* columns past T_out: unused */
 #pragma unroll
             for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -904,6 +917,7 @@ NSR_DEV void conv_pc_body(const nsr_conv_args& a) {
       }
       if (last_chunk && n < items) {
         const nsr_rsrc orr = make_rsrc_uniform(a.out + (int64_t)b * a.C_out * a.T_out, obytes);
+        const bool ragged = (a.T_out & 3) != 0 && t0 + CV_TT > a.T_out; /* wave-uniform */
         nsr_float4 ov[STATS ? 2 : 1][STATS ? 4 : 1];
 #pragma unroll
         for (int m = 0; m < 2; ++m)
@@ -923,9 +937,7 @@ NSR_DEV void conv_pc_body(const nsr_conv_args& a) {
             const float bv = bias_l[min(co, a.C_out - 1)];
             nsr_float4 o = {v[0] + bv, v[1] + bv, v[2] + bv, v[3] + bv};
             if constexpr (RESID) o += rv[m][q];
-            if (t < a.T_out)
-              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, o), orr,
-                                                     ((uint32_t)co * (uint32_t)a.T_out + (uint32_t)t) * 4u, 0, 0);
+            store_quad(orr, ((uint32_t)co * (uint32_t)a.T_out + (uint32_t)t) * 4u, o, a.T_out - t, ragged);
             if constexpr (STATS) ov[m][q] = o;
           }
         if constexpr (STATS)
@@ -1667,14 +1679,7 @@ NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
       ov[m][q] = o;
       const uint32_t co = (uint32_t)(cow + 32 * m + 8 * q + 4 * hl + c4);
       const uint32_t oo = (co * (uint32_t)a.T_out + (uint32_t)t) * 4u;
-      if (nq >= 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, o), orr, oo, 0, 0);
-      if (ragged) {
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-          const float oe = o[e];
-          if (nq < 4 && e < nq) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, oe), orr, oo + 4u * e, 0, 0);
-        }
-      }
+      store_quad(orr, oo, o, nq, ragged);
     }
   if constexpr (STATS)
     emit_rows8(ov, t, t0 + 32 * wt, a.T_out, l32, cow + 4 * hl + c4, a.C_out, (int64_t)b * a.C_out, (a.T_out + 31) >> 5,

@@ -1428,21 +1428,23 @@ nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const 
   const int64_t tiles = (int64_t)cdiv_u(a.T_out, kCvTT) * cdiv_u(a.C_out, kCvCO) * a.B;
   if (tiles > 0x7fffffffLL) return fail(NSR_ERR_UNSUPPORTED, "%s: too many tiles", what);
   const int np = TL <= 72 ? 9 : TL <= 96 ? 12 : 16;  // register pairs per lane: 8 TL <= 64 np
-  // K <= 3 with one channel block each way and 16-byte aligned rows: every weight resident in LDS,
+  // K <= 3 with one channel block each way: every weight resident in LDS,
   // one 512-lane workgroup per CU (producer and consumer waves)
   const int64_t lds_rw = ((int64_t)a.K * kCvCO + 2 * TL) * kCvS * 2;
   const int64_t win = TL + ((-(int64_t)a.padding) & 3);  // staged window from a 16-byte aligned column
-  if (a.C_in <= kCvCI && a.C_out <= kCvCO && a.K <= 3 && win <= 128 && lds_rw <= dm->max_lds && (a.pad_ & 1) &&
-      a.T_in > 0 && a.T_in % 4 == 0 && aligned(a.x, 16)) {
+  // both kernels below form 32-bit offsets of whole 128-channel blocks and 64-column tiles, those past the
+  // output included, and leave dropping them to the range check: they must not wrap
+  const bool fits32 = 4 * (int64_t)cdiv_u(a.C_out, kCvCO) * kCvCO * ((int64_t)a.T_out + kCvTT) <= kConvMaxSlabBytes;
+  if (a.C_in <= kCvCI && a.C_out <= kCvCO && a.K <= 3 && win <= 128 && lds_rw <= dm->max_lds && a.T_in > 0 && fits32) {
     const int64_t groups = std::min<int64_t>(tiles, (int64_t)dm->n_cu);
     if (emitted) *emitted = a.row_part != nullptr;
     return launch(kConvRw[fused][a.residual != nullptr][a.row_part != nullptr][win <= 96 ? 0 : 1], (unsigned)groups,
                   1, 512, (unsigned)lds_rw, stream, params);
   }
-  // any K, C_in in chunks and C_out in blocks of 128, 16-byte aligned rows: weights streamed one tap ahead
+  // any K, C_in in chunks and C_out in blocks of 128: weights streamed one tap ahead
   // through two LDS slots, one 512-lane workgroup per CU (producer and consumer waves)
   const int64_t lds_pc = (2 * TL + 2 * kCvCO) * kCvS * 2 + 4 * (int64_t)a.C_out; /* + the bias as f32 */
-  if (win <= 128 && lds_pc <= dm->max_lds && (a.pad_ & 1) && a.T_in > 0 && a.T_in % 4 == 0 && aligned(a.x, 16)) {
+  if (win <= 128 && lds_pc <= dm->max_lds && a.T_in > 0 && fits32) {
     const int64_t groups = std::min<int64_t>(tiles, (int64_t)dm->n_cu);
     if (emitted) *emitted = a.row_part != nullptr;
     return launch(kConvPc[fused][a.residual != nullptr][a.row_part != nullptr][win <= 96 ? 0 : 1], (unsigned)groups,
@@ -1500,9 +1502,13 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   const int64_t D = (int64_t)(a.K - 1) * a.dilation;
   const int64_t TLe = kCvTW + D + (D & 1);
   // TLe <= 184 leaves 72 ring slots outside a window, which with the 56 rows after the ring stage a 128-row tile.
-  // Below K = 7 the records pass (x read, records written) costs more than the one-launch kernels lose to
-  // their per-element work (measured on MI355X at [8, 128, 115200]: K = 3 about 540 us against 370 us).
-  if (!records || a.K < 7 || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0)
+  // Below K = 7 with one 128-channel block each way the records pass (x read, records written) costs more than
+  // the one-launch kernels lose to their per-element work (measured on MI355X, two dilations of a ResBlock at
+  // K = 3: [4, 128, 57600] 468 us against 595 us on records, [1, 128, 19200] 110 us on both). With more blocks the
+  // one-launch kernel transforms its input once per output block and the records win from K = 3:
+  // [8, 256, 9600] 571 against 639 us, [4, 256, 3200] 147 against 173 us, [1, 256, 3200] 87 against 110 us.
+  const bool blocks1 = a.C_in <= kCvCI && a.C_out <= kCvCO;
+  if (!records || a.K < (blocks1 ? 7 : 3) || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0)
     return conv_launch(fused, a, stream, what, emitted);
   const int64_t Tp = (int64_t)a.T_in + 2 * a.padding;
   const int64_t n_ch = (a.C_in + 127) / 128, n_co = (a.C_out + 127) / 128;
