@@ -9,6 +9,7 @@ is raised.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import re
 from pathlib import Path
 
@@ -142,10 +143,18 @@ def init(code_object_dir: str | None = None) -> None:
     check(lib().nsr_init(code_object_dir.encode() if code_object_dir else None))
 
 
+# torch.cuda.current_stream() builds a Stream object and parses a device on every call, about 3 us; these are the
+# two lookups behind it (the current device's current stream as an integer).
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream) -> int | None:
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return stream.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or _get_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_get_device())
 
 
 def _ptr(t: torch.Tensor | None):
@@ -407,6 +416,7 @@ def _conv_tout(T, K, padding, dilation):
 WS_PACKED_WEIGHTS, WS_IN_STATS, WS_OUT_STATS, WS_RECORDS = 1, 2, 4, 8
 
 
+@functools.lru_cache(maxsize=1024)
 def conv1d_workspace_bytes(B, C_in, C_out, T, K, padding, dilation, parts) -> int:
     """Bytes of device workspace a conv entry point of this shape needs for `parts` (WS_* flags ORed)."""
     n = C.c_int64(0)
