@@ -118,3 +118,42 @@ def test_ragged_rows_from_misaligned_views():
         got, _ = abi.conv1d_f16w_packed_stats(x, wp, None, r, padding=pad, dilation=dil, out=out)
         assert torch.equal(got, want)
         assert torch.equal(ob[:1], keep[:1]) and torch.equal(ob[1 + n:], keep[1 + n:])
+
+
+@pytest.mark.parametrize("C,T,K,dil,pad,res", [
+    (128, 1, 1, 1, 0, False), (16, 63, 1, 1, 5, True), (128, 200, 2, 1, 1, True), (96, 517, 3, 1, 1, True),
+    (128, 64, 3, 32, 32, True),   # the widest halo: 64 columns shared between tiles
+    (128, 131, 3, 5, 70, True),   # padding wider than a tile
+    (64, 1000, 2, 7, 0, False), (128, 40000, 3, 3, 3, True),
+])
+def test_resident_weight_kernel(C, T, K, dil, pad, res):
+    """The K <= 3 kernel's padding, halo and run edges (several tiles per workgroup at T = 40000, B = 2)."""
+    say("conv resident weights", C, T, K, dil, pad, res)
+    g = configs.rng(C + T + K + pad)
+    B, T_out = 2, T + 2 * pad - dil * (K - 1)
+    x = torch.from_numpy(g.standard_normal((B, C, T)).astype(np.float32)).cuda()
+    w = torch.from_numpy((g.standard_normal((C, C, K)) * 0.1).astype(np.float16)).cuda()
+    b = torch.from_numpy(g.standard_normal(C).astype(np.float16)).cuda()
+    r = torch.from_numpy(g.standard_normal((B, C, T_out)).astype(np.float32)).cuda() if res else None
+    xp = torch.nn.functional.pad(x.double(), (pad, pad))
+    ref = b.double()[None, :, None].expand(B, -1, T_out).clone()
+    mag = torch.zeros_like(ref)
+    for k in range(K):
+        for i in range(B):
+            s = xp[i, :, k * dil:k * dil + T_out].contiguous()
+            ref[i] += w[:, :, k].double().contiguous() @ s
+            mag[i] += w[:, :, k].double().abs().contiguous() @ s.abs()
+    if res:
+        ref, mag = ref + r.double(), mag + r.double().abs()
+    # |y - hi - lo| <= 2^-22 |y|, C K products summed in f32
+    bar = (2.0 ** -22 + C * K * 2.0 ** -24) * mag + 2.0 ** -23 * ref.abs() + 1e-30
+    wp = abi.conv1d_pack_f16(w)
+    o = abi.conv1d_f16w_packed(x, wp, b, r, padding=pad, dilation=dil)
+    worst = float(((o.double() - ref).abs() / bar).max())
+    assert worst <= 1.0, f"{worst:.2f} of the bar"
+    o2, st = abi.conv1d_f16w_packed_stats(x, wp, b, r, padding=pad, dilation=dil)
+    assert torch.equal(o, o2)
+    d = o.double().view(B * C, T_out)
+    spread = torch.sqrt(d.var(-1, unbiased=False) + 1e-5)
+    assert bool(((st[:, 0].double() - d.mean(-1)).abs() <= 1e-5 * torch.maximum(d.mean(-1).abs(), spread)).all())
+    assert bool(((st[:, 1].double() * spread - 1.0).abs() <= 1e-5).all())
