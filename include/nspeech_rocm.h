@@ -195,8 +195,8 @@ nsr_status nsr_kv_cache_append(const void* new_kv, void* cache, nsr_dtype dtype,
  * gamma/beta/alpha have param_dtype F32 or F16. gamma_bstride/beta_bstride:
  * elements between batches of gamma/beta (0 = shared over the batch, C =
  * per batch). alpha is per channel [C].
- * While a row fits on chip (16-byte aligned rows up to T = 118784, other rows
- * up to about 65k elements) x is read from HBM once and the statistics are
+ * While a row fits on chip (x and out 16-byte aligned: T up to about 118,790;
+ * other addresses: up to about 65k elements) x is read from HBM once and the statistics are
  * two passes over the on-chip row in f32 (the mean, then centred sums that
  * also correct the mean). Longer rows take a kernel that reads each row
  * twice (f64 sums, then the output; no scratch memory).

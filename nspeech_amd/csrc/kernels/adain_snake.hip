@@ -109,7 +109,7 @@ NSR_DEV float sum4(nsr_float4 d) { return (d.x + d.y) + (d.z + d.w); }
  * slot's output is stored (stores and refills in batches of 8 slots), so on a
  * CU the reads of the next row overlap the writes of the current one, and HBM traffic stays the algorithmic
  * 8 bytes per element (x read once, out written once). */
-template <int BLOCK, int NV, int NL, bool TL = false>
+template <int BLOCK, int NV, int NL, bool TL = false, bool U = false>
 NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
   NSR_NO_CONTRACT
   constexpr int NW = BLOCK / 64;
@@ -139,8 +139,32 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
     }
   }
   const int64_t T = a.T;
-  const int nch = (int)(T >> 2);
-  const uint32_t rbytes = (uint32_t)(T * 4);
+  /* U (T % 4 != 0, x and out 16-byte aligned): the slots hold the row's interior 16-byte chunks, those of the
+   * tensor's grid wholly inside it; the up to 4 + 4 elements of the first and last chunk go one each to the last 8
+   * lanes of the workgroup. */
+  struct row_geom {
+    int64_t a0;  /* first element of the row's first chunk */
+    int lo, nchunk;
+  };
+  auto geom = [&](int64_t r) {
+    const int64_t s0 = r * T;
+    row_geom g;
+    g.a0 = U ? s0 & ~(int64_t)3 : s0;
+    g.lo = U ? (int)(s0 & 3) : 0;
+    g.nchunk = U ? (int)((g.lo + T + 3) >> 2) : (int)(T >> 2);
+    return g;
+  };
+  /* first element and bytes of the slots' range */
+  auto slots_at = [&](const row_geom& g) { return U ? g.a0 + 4 : g.a0; };
+  auto slots_n = [&](const row_geom& g) { return U ? g.nchunk - 2 : g.nchunk; };
+  const int eq = tid - (BLOCK - 8);
+  auto edge_at = [&](const row_geom& g) { return (int64_t)(eq >= 4 ? 4 * (g.nchunk - 1) : 0) + (eq & 3); };
+  auto edge_ok = [&](const row_geom& g) {
+    const int64_t e = edge_at(g);
+    return U && eq >= 0 && e >= g.lo && e < g.lo + T;
+  };
+  row_geom rg = geom(row);
+  float xe = edge_ok(rg) ? a.x[rg.a0 + edge_at(rg)] : 0.f;
   const uint32_t voff = (uint32_t)tid * 16u;
   /* LDS slots of this wave: base address wave-uniform (an SGPR, M0 per load);
    * lane i of the wave lands at base + 16 i, i.e. at lds_x[m * BLOCK + tid] */
@@ -149,7 +173,8 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
   /* slot k of this lane lies inside the row iff k < nvalid (tested for the
    * last MK slots only; a per-slot lane mask for every slot would be kept in
    * SGPR pairs across the row loop) */
-  const int nvalid = nch > tid ? (nch - tid + BLOCK - 1) / BLOCK : 0;
+  auto count_valid = [&](int nch) { return nch > tid ? (nch - tid + BLOCK - 1) / BLOCK : 0; };
+  int nvalid = count_valid(slots_n(rg));
   auto valid = [&](int k) { return k < NS - MK || k < nvalid; };
   const nsr_float4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
@@ -172,7 +197,7 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
   /* first row: every slot's load, then the parameters */
   nsr_float4 v[NV];
   {
-    const nsr_rsrc xr = make_rsrc(a.x + row * T, rbytes);
+    const nsr_rsrc xr = make_rsrc(a.x + slots_at(rg), (uint32_t)slots_n(rg) * 16u);
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = vload(xr, k, voff, (uint32_t)(k * BLOCK * 16));
 #pragma unroll
@@ -194,7 +219,7 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
     }
 
     /* one pass: sum and sum of squares */
-    float s = 0.f, q = 0.f;
+    float s = xe, q = xe * xe; /* 0 on lanes without an edge element */
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       if (valid(k)) {
@@ -224,7 +249,8 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
     float vshift = mean, lbase = 0.f;
     if (4.0f * mean * mean > var) {
       /* second pass: centred sums; the VGPR slots keep x - mean (0 outside the row) */
-      float s1 = 0.f, s2 = 0.f;
+      const float de = edge_ok(rg) ? xe - mean : 0.f;
+      float s1 = de, s2 = de * de;
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
         const nsr_float4 d = v[k] - mean;
@@ -270,8 +296,13 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
       }
       pr = adain_params_load(a, pdt, bn, cn);
     }
-    const nsr_rsrc orr = make_rsrc(a.out + row * T, rbytes);
-    const nsr_rsrc xn = make_rsrc(a.x + (more ? next : row) * T, more ? rbytes : 0u);
+    const row_geom ng = geom(more ? next : row);
+    const nsr_rsrc orr = make_rsrc(a.out + slots_at(rg), (uint32_t)slots_n(rg) * 16u);
+    const nsr_rsrc xn = make_rsrc(a.x + slots_at(ng), more ? (uint32_t)slots_n(ng) * 16u : 0u);
+    if constexpr (U) {
+      if (edge_ok(rg)) a.out[rg.a0 + edge_at(rg)] = snake_eval(__builtin_fmaf(xe - lbase, A, Bc), sc);
+      xe = more && edge_ok(ng) ? a.x[ng.a0 + edge_at(ng)] : 0.f;
+    }
     /* slot offsets are formed from a fresh copy of the lane offset and an
      * opaque zero each row: as loop invariants the compiler would keep all
      * NS of them live in registers across the loop */
@@ -312,6 +343,8 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
     });
     if (!more) break;
     row = next;
+    rg = ng;
+    if constexpr (U) nvalid = count_valid(slots_n(rg));
   }
   if constexpr (TL) {
     NSR_WAIT_VMCNT(0); /* this wave's last stores have completed */
@@ -387,6 +420,44 @@ NSR_ADAIN_ROW(512, 36, 19)
 NSR_ADAIN_ROW(512, 37, 19)
 NSR_ADAIN_ROW(512, 38, 19)
 NSR_ADAIN_ROW(512, 39, 19)
+
+/* Rows past T = 8192 that are not a multiple of 4 long. VGPR slots up to 19, 19 LDS slots and an even number of
+ * VGPR slots beyond. What bounds it is what bounds the aligned rows; the chunks stay on the 16-byte grid, so no
+ * access is split, and the edges cost one load and one store. Measured on MI355X, graph replays of one call, against
+ * the kernels these rows took before (one workgroup per row; past T = 65,538 two reads of the row):
+ * [8, 128, 115201] 210 against 554 us ([8, 128, 115200] on the aligned kernel: 185), [1, 128, 115201] 31 against 130,
+ * [4, 128, 57601] 51 against 53.5, [8, 128, 28801] 47.5 against 52.0. */
+#define NSR_ADAIN_ROW_U(NV, NL)                                                             \
+  extern "C" __global__ void __launch_bounds__(512)                                        \
+      nsrk_adain_rowu_b512_v##NV##_l##NL(const nsr_adain_args a, const int pdt) {          \
+    adain_row<512, NV, NL, false, true>(a, pdt);                                           \
+  }
+NSR_ADAIN_ROW_U(6, 0)
+NSR_ADAIN_ROW_U(8, 0)
+NSR_ADAIN_ROW_U(10, 0)
+NSR_ADAIN_ROW_U(12, 0)
+NSR_ADAIN_ROW_U(16, 0)
+NSR_ADAIN_ROW_U(20, 0)
+NSR_ADAIN_ROW_U(2, 19)
+NSR_ADAIN_ROW_U(4, 19)
+NSR_ADAIN_ROW_U(6, 19)
+NSR_ADAIN_ROW_U(8, 19)
+NSR_ADAIN_ROW_U(10, 19)
+NSR_ADAIN_ROW_U(12, 19)
+NSR_ADAIN_ROW_U(14, 19)
+NSR_ADAIN_ROW_U(16, 19)
+NSR_ADAIN_ROW_U(18, 19)
+NSR_ADAIN_ROW_U(20, 19)
+NSR_ADAIN_ROW_U(22, 19)
+NSR_ADAIN_ROW_U(24, 19)
+NSR_ADAIN_ROW_U(26, 19)
+NSR_ADAIN_ROW_U(28, 19)
+NSR_ADAIN_ROW_U(30, 19)
+NSR_ADAIN_ROW_U(32, 19)
+NSR_ADAIN_ROW_U(34, 19)
+NSR_ADAIN_ROW_U(36, 19)
+NSR_ADAIN_ROW_U(38, 19)
+NSR_ADAIN_ROW_U(39, 19)
 
 /* The c4b row kernel (T of 56-57 slots) with the timeline stamps, for the measurement entry point
  * nsr_calib_adain_timeline: where in a call each workgroup and wave spends its time. */
@@ -525,7 +596,9 @@ NSR_ADAIN_RES_U(512, 32)
  * and last chunk may be partial and are taken one element per lane by the
  * last 16 lanes, the interior chunks 1..nch-2 are spread as
  * j = 1 + tid + BLOCK k with clamped, branch-free loads. out must share x's offset within 16 bytes (checked by
- * the host). Two-pass statistics over the registers, as the f32 kernels. */
+ * the host). One-pass statistics, the centred pass when 4 mean^2 > var, as the
+ * f32 kernels ([4, 128, 57601]: 25.8 us against 28.8 us per graph replay with
+ * two-pass statistics over widened values; [8, 128, 115201] 109 against 119). */
 /* pointers rebuilt from integer addresses are generic (flat accesses, which
  * count against both memory counters); these keep them global */
 typedef __attribute__((address_space(1))) uint16_t nsr_gh;
@@ -540,7 +613,7 @@ template <int BLOCK, int NV>
 NSR_DEV void adain_row_f16(const nsr_adain_h_args& a, int pdt) {
   NSR_NO_CONTRACT
   constexpr int NW = BLOCK / 64;
-  __shared__ float red[3 * NW]; /* [0, NW): the mean's sums, [NW, 3 NW): the centred sums */
+  __shared__ float red[4 * NW]; /* [0, 2 NW): the one-pass sums, [2 NW, 4 NW): the centred sums */
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   if (row >= a.n_rows) return; /* whole workgroup: the grid is one per row */
@@ -581,62 +654,93 @@ NSR_DEV void adain_row_f16(const nsr_adain_h_args& a, int pdt) {
   row_bc32(row, a.C, bi, ci);
   const adain_raw pr = adain_params_load(a, pdt, bi, ci);
 
-  float sum = xe;
+  /* one pass (sum and sum of squares straight from the packed halves, products exact in f32), the centred pass
+   * when 4 mean^2 > var, as adain_row_h; slots outside the interior hold zeros */
+  typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+  const h2_t one = {(_Float16)1.0f, (_Float16)1.0f};
+  float sum = xe, ssq = xe * xe;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    float f[8];
-    unpack16<DT_F16>(v[k], f);
-    sum += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
-  }
-  const float mean = block_sum<NW, false>(sum, red) * a.inv_t;
-
-  /* the chunks stay raw (4 VGPRs each) between passes: an empty asm that
-   * "modifies" them stops the compiler keeping their unpacked floats (8) live */
+    float t = 0.f, u = 0.f;
 #pragma unroll
-  for (int k = 0; k < NV; ++k) asm volatile("" : "+v"(v[k]));
-  /* centred sums; slots outside the interior hold zeros and are weighted out */
-  float sq = 0.f, sd = 0.f;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int j = jbase + BLOCK * k;
-    float f[8], q = 0.f, t = 0.f;
-    unpack16<DT_F16>(v[k], f);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float d = f[e] - mean;
-      q = __builtin_fmaf(d, d, q);
-      t += d;
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t wi = v[k][i]; /* a named copy: a bit_cast of the vector element itself reads element 0 */
+      const h2_t hw = __builtin_bit_cast(h2_t, wi);
+      t = __builtin_amdgcn_fdot2(hw, one, t, false);
+      u = __builtin_amdgcn_fdot2(hw, hw, u, false);
     }
-    sq += j <= jmax ? q : 0.f;
-    sd += j <= jmax ? t : 0.f;
+    sum += t;
+    ssq += u;
   }
-  if (eok) {
-    const float d = xe - mean;
-    sq = __builtin_fmaf(d, d, sq);
-    sd += d;
+  block_sum2<NW, false>(sum, ssq, red);
+  const float mean = sum * a.inv_t;
+  float var = __builtin_fmaf(-mean, mean, ssq * a.inv_t);
+  float sub = 0.f, vshift = mean; /* the output is (x - sub) A + Bc, Bc = beta - vshift A */
+  if (4.0f * mean * mean > var) {
+    /* centred sums; slots outside the interior are weighted out */
+    float sq = 0.f, sd = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int j = jbase + BLOCK * k;
+      float f[8], q = 0.f, t = 0.f;
+      unpack16<DT_F16>(v[k], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = f[e] - mean;
+        q = __builtin_fmaf(d, d, q);
+        t += d;
+      }
+      sq += j <= jmax ? q : 0.f;
+      sd += j <= jmax ? t : 0.f;
+    }
+    if (eok) {
+      const float d = xe - mean;
+      sq = __builtin_fmaf(d, d, sq);
+      sd += d;
+    }
+    block_sum2<NW, false>(sq, sd, red + 2 * NW);
+    vshift = sd * a.inv_t;
+    sub = mean;
+    var = __builtin_fmaf(-vshift, sd, sq) * a.inv_t;
   }
-  block_sum2<NW, false>(sq, sd, red + NW);
-  const float c = sd * a.inv_t;
-  const float var = fmaxf(__builtin_fmaf(-c, sd, sq) * a.inv_t, 0.0f);
+  var = fmaxf(var, 0.0f);
   const float rstd = __builtin_amdgcn_rsqf(var + a.eps); /* v_rsq_f32, about 1 ulp */
   float gam, bet, alp;
   adain_params_cvt(pr, pdt, gam, bet, alp);
   const float A = (gam + 1.0f) * rstd;
-  const float Bc = __builtin_fmaf(-c, A, bet); /* (x - mean - c) A + beta */
+  const float Bc = __builtin_fmaf(-vshift, A, bet);
   const snake_consts_h sc = make_snake_consts_h(alp); /* f16 output */
 
+  /* the chunks stay raw (4 VGPRs each): an empty asm that "modifies" them stops the compiler keeping their
+   * unpacked floats (8) live across the passes */
 #pragma unroll
   for (int k = 0; k < NV; ++k) asm volatile("" : "+v"(v[k]));
+  if (sub == 0.f) { /* uniform: x A + Bc straight from each packed half (v_fma_mix_f32) */
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int j = jbase + BLOCK * k;
-    float f[8], o[8];
-    unpack16<DT_F16>(v[k], f);
+    for (int k = 0; k < NV; ++k) {
+      const int j = jbase + BLOCK * k;
+      float o[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = snake_eval(__builtin_fmaf(f[e] - mean, A, Bc), sc);
-    if (j <= jmax) st16g(ob + 8 * (int64_t)j, pack16<DT_F16>(o));
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t wi = v[k][i];
+        const h2_t hw = __builtin_bit_cast(h2_t, wi);
+        o[2 * i] = snake_eval(__builtin_fmaf((float)hw.x, A, Bc), sc);
+        o[2 * i + 1] = snake_eval(__builtin_fmaf((float)hw.y, A, Bc), sc);
+      }
+      if (j <= jmax) st16g(ob + 8 * (int64_t)j, pack16<DT_F16>(o));
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int j = jbase + BLOCK * k;
+      float f[8], o[8];
+      unpack16<DT_F16>(v[k], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = snake_eval(__builtin_fmaf(f[e] - sub, A, Bc), sc);
+      if (j <= jmax) st16g(ob + 8 * (int64_t)j, pack16<DT_F16>(o));
+    }
   }
-  if (eok) ob[eidx] = (uint16_t)f32_to_f16_bits(snake_eval(__builtin_fmaf(xe - mean, A, Bc), sc));
+  if (eok) ob[eidx] = (uint16_t)f32_to_f16_bits(snake_eval(__builtin_fmaf(xe - sub, A, Bc), sc));
 }
 
 #define NSR_ADAIN_F16(BLOCK, NV)                                                        \

@@ -705,6 +705,7 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
   const bool is_aligned = aligned(x, 16) && aligned(out, 16) && (T % 4 == 0);
   KId kid = K_NONE;
   unsigned block = 0, lds = 0;
+  bool persistent = is_aligned;
   if (is_aligned) {
     // Row kernel: BLOCK-wide slots of 16-byte chunks, NV in VGPRs + NL in LDS. The kernel masks only its
     // last four slots at the row end, so the first NV + NL - 4 slots must lie inside every row.
@@ -755,7 +756,46 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
     const int ns = nv + nl;
     if (block && (int64_t)(ns - std::min(ns, 4)) * block > nch)
       return fail(NSR_ERR_HIP, "adain_snake: internal error: row kernel slots do not fit T=%lld", (long long)T);
-  } else {
+  } else if (aligned(x, 16) && aligned(out, 16) && T > 8 * 1024 && (T + 6) / 4 - 2 <= 512 * (39 + 19)) {
+    // Rows of T % 4 != 0 elements past the 256-lane kernels: the row kernel over the interior chunks of the 16-byte
+    // grid, edges by element (ceil(T / 4) - 2 to (T + 6) / 4 - 2 interior chunks, by the row's start). Against the
+    // one-row-per-workgroup kernel below and the two-read kernel past its 32 slots, us per graph
+    // replay: [8, 128, 12001] 24.1 / 24.0, [8, 128, 28801] 47.5 / 52.0, [4, 128, 57601] 51.0 / 53.5,
+    // [8, 128, 115201] 210 / 554, [1, 128, 115201] 31 / 130.
+    const int64_t nch = (T + 6) / 4 - 2, nmin = (T + 3) / 4 - 2;
+    int nv = 0, nl = 0;
+    if (nch <= 512 * 19) {
+      static const int opts[] = {6, 8, 10, 12, 16, 20};
+      static const KId ids[] = {K_nsrk_adain_rowu_b512_v6_l0,  K_nsrk_adain_rowu_b512_v8_l0,  K_nsrk_adain_rowu_b512_v10_l0,
+                                K_nsrk_adain_rowu_b512_v12_l0, K_nsrk_adain_rowu_b512_v16_l0, K_nsrk_adain_rowu_b512_v20_l0};
+      for (int i = 0; i < 6 && !nv; ++i)
+        if (512LL * opts[i] >= nch) {
+          nv = opts[i];
+          kid = ids[i];
+        }
+    } else {
+      static const KId ids[] = {
+        K_nsrk_adain_rowu_b512_v2_l19, K_nsrk_adain_rowu_b512_v4_l19, K_nsrk_adain_rowu_b512_v6_l19,
+        K_nsrk_adain_rowu_b512_v8_l19, K_nsrk_adain_rowu_b512_v10_l19, K_nsrk_adain_rowu_b512_v12_l19,
+        K_nsrk_adain_rowu_b512_v14_l19, K_nsrk_adain_rowu_b512_v16_l19, K_nsrk_adain_rowu_b512_v18_l19,
+        K_nsrk_adain_rowu_b512_v20_l19, K_nsrk_adain_rowu_b512_v22_l19, K_nsrk_adain_rowu_b512_v24_l19,
+        K_nsrk_adain_rowu_b512_v26_l19, K_nsrk_adain_rowu_b512_v28_l19, K_nsrk_adain_rowu_b512_v30_l19,
+        K_nsrk_adain_rowu_b512_v32_l19, K_nsrk_adain_rowu_b512_v34_l19, K_nsrk_adain_rowu_b512_v36_l19,
+        K_nsrk_adain_rowu_b512_v38_l19,
+        K_nsrk_adain_rowu_b512_v39_l19};
+      nl = 19;
+      const int need = (int)((nch + 511) / 512) - nl; /* 1 .. 39 */
+      nv = need >= 39 ? 39 : (need + 1) / 2 * 2;
+      kid = ids[nv == 39 ? 19 : nv / 2 - 1];
+      lds = (unsigned)(nl * 512 * 16);
+    }
+    if (lds + 1024 <= (unsigned)dm->max_lds) block = 512;
+    // the kernel masks only its last four slots at the row end
+    if (block && (int64_t)(nv + nl - 4) * 512 > nmin)
+      return fail(NSR_ERR_HIP, "adain_snake: internal error: row kernel slots do not fit T=%lld", (long long)T);
+    persistent = true;
+  }
+  if (!is_aligned && !block) {
     // Unaligned rows: interior chunks 1..nch-2 resident in VGPRs, edges by element.
     const int64_t need = (T + 6) / 4 - 2 > 0 ? (T + 6) / 4 - 2 : 0;
     static const int small[] = {1, 2, 3, 4, 5, 6, 8};
@@ -783,7 +823,7 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
     // as many workgroups as fit on the device at once, each walking rows with the grid as stride (one per row
     // when they all fit): a row kernel that fills a CU then overlaps the next row's reads with its writes
     unsigned grid = (unsigned)n_rows;
-    if (is_aligned) grid = (unsigned)std::min<int64_t>(n_rows, (int64_t)occupancy(dm, kid, block, lds) * dm->n_cu);
+    if (persistent) grid = (unsigned)std::min<int64_t>(n_rows, (int64_t)occupancy(dm, kid, block, lds) * dm->n_cu);
     return launch(kid, grid, 1, block, lds, stream, params);
   }
   // Rows past the on-chip budget: statistics over one read, then a second read to apply (persistent grid,
