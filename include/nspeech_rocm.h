@@ -464,7 +464,7 @@ nsr_status nsr_adain_snake_conv1d_f32(const float* x, const void* gamma, const v
  * each x row) replaces the statistics pass over x when not NULL (the
  * previous stage's out_stats); out_stats, when not NULL, receives the same
  * pair for each row of out (after bias and residual), for the next stage's
- * AdaIN. With 16-byte aligned rows the conv's epilogue produces them from
+ * AdaIN. The conv's epilogue produces them from
  * registers (per 32-column block count, mean and M2, merged per row by
  * Chan's pairwise formula) instead of a second read of out. Workspace:
  * NSR_WS_IN_STATS when x_stats is NULL, NSR_WS_OUT_STATS when out_stats is
