@@ -1027,7 +1027,7 @@ struct cv_trans {
  * lies past T_out, and the statistics need no column masks (the masked form
  * and the dispatch between the two would not fit the kernel's registers). */
 template <bool RESID, bool STATS = false, bool FULL32 = false>
-NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8_t* wf) {
+NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8_t* wf, int n_tiles) {
   extern __shared__ __attribute__((aligned(16))) uint8_t cv_ring[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); /* wave-uniform: role and tile math in SALU */
@@ -1036,7 +1036,6 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
   const int Tp = a.T_out + D;                       /* records per (batch, channel chunk) */
   const int n_t = (a.T_out + CV_TW - 1) / CV_TW, n_co = (a.C_out + CV_CO - 1) / CV_CO;
   const int n_ch = (a.C_in + CV_CI - 1) / CV_CI;
-  const int n_tiles = n_t * n_co * a.B;
 
   /* XCD-aware: XCD x (blocks x, x + 8, ...) takes an eighth of the tiles; each workgroup a contiguous run */
   const int G = (int)gridDim.x;
@@ -1494,23 +1493,24 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
 
 #define NSR_CONV_PR1(NAME, RESID)                                                                    \
   extern "C" __global__ void __launch_bounds__(512, 1)                                              \
-      NAME(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {                           \
-    conv_pr_body<RESID>(a, xs, wf);                                                                 \
+      NAME(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf, const int n_tiles) {                           \
+    conv_pr_body<RESID>(a, xs, wf, n_tiles);                                                                 \
   }                                                                                                 \
   extern "C" __global__ void __launch_bounds__(512, 1)                                              \
-      NAME##_st(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {                      \
-    conv_pr_body<RESID, true>(a, xs, wf);                                                           \
+      NAME##_st(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf, const int n_tiles) {                      \
+    conv_pr_body<RESID, true>(a, xs, wf, n_tiles);                                                           \
   }                                                                                                 \
   extern "C" __global__ void __launch_bounds__(512, 1)                                              \
-      NAME##_st32(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {                    \
-    conv_pr_body<RESID, true, true>(a, xs, wf);                                                     \
+      NAME##_st32(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf, const int n_tiles) {                    \
+    conv_pr_body<RESID, true, true>(a, xs, wf, n_tiles);                                                     \
   }
 NSR_CONV_PR1(nsrk_conv1d_pr_f16x2, false)
 NSR_CONV_PR1(nsrk_conv1d_pr_res_f16x2, true)
 
 /* ------------------------------------- conv on records, small output tiles -- */
 
-/* The record kernel for outputs with too few 128 x 128 tiles to fill the chip: one 256-lane workgroup per
+/* The record kernel for outputs with too few 128 x 128 tiles to fill the chip, and for the rest of one that
+ * fills it several times (column tiles from ct0 on): one 256-lane workgroup per
  * tile of 64 MT channels x 64 columns, 2 x 2 waves of 32 MT channels x 32 columns, several workgroups per CU
  * where LDS and registers allow. A workgroup copies its window of 64 + (K - 1) dilation records of one
  * channel chunk straight to LDS (buffer_load ... lds) and then only multiplies:
@@ -1527,7 +1527,7 @@ NSR_CONV_PR1(nsrk_conv1d_pr_res_f16x2, true)
  * three steps ahead. */
 #define CV_PS 1040
 template <int MT, bool RESID, bool STATS>
-NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8_t* wf) {
+NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8_t* wf, int ct0) {
   extern __shared__ __attribute__((aligned(16))) uint8_t cv_ps[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wco = wave >> 1, wt = wave & 1;
@@ -1538,8 +1538,9 @@ NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
 
   /* tiles with the channel block slowest, an eighth of them per XCD: an XCD's L2 then holds one block's weights */
   const int tile = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
-  const int tb_all = n_t * a.B, cb = tile / tb_all, rt = tile - cb * tb_all;
-  const int b = rt / n_t, t0 = (rt - b * n_t) * CV_TT, co0 = cb * 64 * MT;
+  const int n_ct = n_t * a.B - ct0; /* column tiles ct0 .. of all batches */
+  const int cb = tile / n_ct, ct = ct0 + tile - cb * n_ct;
+  const int b = ct / n_t, t0 = (ct - b * n_t) * CV_TT, co0 = cb * 64 * MT;
   const int cow = co0 + 32 * MT * wco;               /* the wave's first channel */
   const int t = t0 + 32 * wt + 4 * (l32 >> 2);       /* this lane's column quad after the quad transpose */
 
@@ -1688,12 +1689,12 @@ NSR_DEV void conv_ps_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
 
 #define NSR_CONV_PS1(NAME, MT, RESID)                                                                \
   extern "C" __global__ void __launch_bounds__(256, 2)                                              \
-      NAME(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {           \
-    conv_ps_body<MT, RESID, false>(a, xs, wf);                                                \
+      NAME(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf, const int ct0) {           \
+    conv_ps_body<MT, RESID, false>(a, xs, wf, ct0);                                                \
   }                                                                                                 \
   extern "C" __global__ void __launch_bounds__(256, 2)                                              \
-      NAME##_st(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf) {      \
-    conv_ps_body<MT, RESID, true>(a, xs, wf);                                                 \
+      NAME##_st(const nsr_conv_args a, const uint8_t* xs, const uint8_t* wf, const int ct0) {      \
+    conv_ps_body<MT, RESID, true>(a, xs, wf, ct0);                                                 \
   }
 NSR_CONV_PS1(nsrk_conv1d_ps1_f16x2, 1, false)
 NSR_CONV_PS1(nsrk_conv1d_ps1_res_f16x2, 1, true)

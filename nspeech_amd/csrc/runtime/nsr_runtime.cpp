@@ -1576,21 +1576,36 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   // 200 187 / 206 / 191, 226 149 / 151 / 145, 280 386 / 322 / 338, 302 241 / 211 / 219, 452 286 / 300 / 298.
   // MT = 1 (four times the tiles) while they fit one per CU, and past one round of the large tiles.
   const int64_t rounds = (tiles + dm->n_cu - 1) / dm->n_cu;
-  if (rounds <= 2 && 10 * tiles <= 7 * rounds * dm->n_cu) {
-    static const KId ps[2][2][2] = {{{K_nsrk_conv1d_ps1_f16x2, K_nsrk_conv1d_ps1_f16x2_st},
-                                     {K_nsrk_conv1d_ps1_res_f16x2, K_nsrk_conv1d_ps1_res_f16x2_st}},
-                                    {{K_nsrk_conv1d_ps2_f16x2, K_nsrk_conv1d_ps2_f16x2_st},
-                                     {K_nsrk_conv1d_ps2_res_f16x2, K_nsrk_conv1d_ps2_res_f16x2_st}}};
-    const int mt = 4 * tiles <= dm->n_cu || rounds == 2 ? 1 : 2;
+  static const KId ps[2][2][2] = {{{K_nsrk_conv1d_ps1_f16x2, K_nsrk_conv1d_ps1_f16x2_st},
+                                   {K_nsrk_conv1d_ps1_res_f16x2, K_nsrk_conv1d_ps1_res_f16x2_st}},
+                                  {{K_nsrk_conv1d_ps2_f16x2, K_nsrk_conv1d_ps2_f16x2_st},
+                                   {K_nsrk_conv1d_ps2_res_f16x2, K_nsrk_conv1d_ps2_res_f16x2_st}}};
+  // the small-tile kernel over the column tiles of 64 from ct0 on (batches in a row)
+  auto small_tiles = [&](int mt, int ct0) {
     const unsigned slots = D <= 32 ? 48 : 64;  // record slots in LDS: 64 + D <= 2 * slots
-    const int64_t grid = (int64_t)cdiv_u(a.T_out, 64) * cdiv_u(a.C_out, 64 * mt) * a.B;
-    return launch(ps[mt - 1][a.residual != nullptr][stats], (unsigned)grid, 1, 256, slots * 1040, stream, pp);
-  }
+    const int64_t grid = ((int64_t)cdiv_u(a.T_out, 64) * a.B - ct0) * cdiv_u(a.C_out, 64 * mt);
+    void* pq[] = {&a, &xs, &wf, &ct0};
+    return launch(ps[mt - 1][a.residual != nullptr][stats], (unsigned)grid, 1, 256, slots * 1040, stream, pq);
+  };
+  if (rounds <= 2 && 10 * tiles <= 7 * rounds * dm->n_cu)
+    return small_tiles(4 * tiles <= dm->n_cu || rounds == 2 ? 1 : 2, 0);
+  // A last round that fills at most a third of the chip goes to the small-tile kernel in a launch of its own
+  // (whole columns of channel blocks). Measured, us per ResBlock, one launch / two: [8, 256, 4200] K = 11 (528
+  // tiles) 568 / 534, [5, 128, 26400] K = 7 (1035) 474 / 467, [4, 128, 57601] K = 11 (1804) 1405 / 1390.
+  int n_tiles = (int)tiles;
+  const int64_t rest = tiles % dm->n_cu;
+  // (the small-tile kernel's 32-bit offsets of whole channel blocks must not wrap)
+  if (rounds > 2 && rest > 0 && 3 * rest <= dm->n_cu && 4 * n_co * kCvCO * ((int64_t)a.T_out + kCvTW) <= kConvMaxSlabBytes)
+    n_tiles = (int)((tiles - rest) / n_co * n_co);
   // one workgroup per CU, a multiple of 8 (the kernel's XCD split), never fewer than there are tiles below that:
   // rounded down, 151 tiles gave some of 144 workgroups a second tile (256 against 193 us per ResBlock)
   const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((tiles + 7) / 8 * 8, dm->n_cu >= 8 ? dm->n_cu / 8 * 8 : dm->n_cu));
   const int kv = stats ? (a.T_out % 32 == 0 ? 2 : 1) : 0;
-  return launch(ids[a.residual != nullptr][kv], (unsigned)grid, 1, 512, kCvRingLds, stream, pp);
+  void* pr[] = {&a, &xs, &wf, &n_tiles};
+  st = launch(ids[a.residual != nullptr][kv], (unsigned)grid, 1, 512, kCvRingLds, stream, pr);
+  if (st != NSR_OK || n_tiles == tiles) return st;
+  const int64_t col = n_tiles / n_co, n_t = cdiv_u(a.T_out, kCvTW);  // the first column of 128 left: (batch, tile)
+  return small_tiles(1, (int)(col / n_t * cdiv_u(a.T_out, 64) + 2 * (col % n_t)));
 }
 
 // Launch a conv and leave the per-(b, co) statistics of its output in row_stats ([B*C_out][2]: mean,

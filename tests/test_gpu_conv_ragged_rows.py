@@ -51,6 +51,9 @@ def _reference(x, gam, bet, alp, w, bias, res, pad, dil):
     (3, 64, 96, 1001, 8, 1, True),      # odd (K - 1) dilation
     (1, 128, 128, 19201, 11, 5, True),  # many tiles per workgroup are not reached; tiles past one per CU are below
     (2, 128, 128, 19203, 7, 5, True),
+    (3, 128, 128, 128 * 257 - 63, 7, 1, True),   # three rounds of tiles and a rest of 3, a half tile at each row's end
+    (2, 256, 256, 128 * 130 + 5, 7, 3, True),    # two channel blocks, a rest of 12 across the last batch
+    (3, 128, 128, 128 * 171 + 32, 7, 1, False),  # a rest that starts inside the last batch, whole 32-column blocks
     (1, 64, 64, 601, 5, 2, True),       # K < 7: the one-launch kernels
     (2, 128, 128, 1003, 3, 5, True),
     (1, 128, 128, 19201, 3, 1, False),
