@@ -83,6 +83,50 @@ NSR_DEV float sumsq4(nsr_float4 d, float sq) {
 
 NSR_DEV float sum4(nsr_float4 d) { return (d.x + d.y) + (d.z + d.w); }
 
+/* mean as an unevaluated f32 pair (hi + lo) and 1 / sqrt(var + eps) */
+NSR_DEV void row_moments(double s1, double s2, int64_t T, float eps, float& mhi, float& mlo, float& rstd) {
+  const double mean = s1 / (double)T;
+  double var = s2 / (double)T - mean * mean;
+  var = var > 0.0 ? var : 0.0;
+  mhi = (float)mean;
+  mlo = (float)(mean - (double)mhi);
+  rstd = 1.0f / sqrtf((float)var + eps);
+}
+
+/* A value pair summed over the workgroup in f64; `red` holds 2 NW doubles. No trailing barrier: the caller
+ * alternates two buffers, as for block_sum2 without REUSE. */
+template <int NW>
+NSR_DEV void block_sum2_f64(double& a, double& b, double* red) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    a += __shfl_xor(a, off);
+    b += __shfl_xor(b, off);
+  }
+  const int wid = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    red[wid] = a;
+    red[NW + wid] = b;
+  }
+  __syncthreads();
+  a = 0.0;
+  b = 0.0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    a += red[w];
+    b += red[NW + w];
+  }
+}
+
+/* The four elements of a chunk added to f64 sums of x and x^2. */
+NSR_DEV void sums4_f64(nsr_float4 x, double& s, double& q) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const double d = (double)x[e];
+    s += d;
+    q = __builtin_fma(d, d, q);
+  }
+}
+
 /* ------------------------------------------------------------ row kernel -- */
 
 /* Rows of a workgroup: row = blockIdx.x, + gridDim.x, ... The host launches
@@ -118,9 +162,13 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
    * with (NS - MK) * BLOCK <= T / 4 */
   constexpr int MK = NS < 4 ? NS : 4;
   extern __shared__ nsr_float4 lds_x[];
-  /* two block-sum buffers of 2 NW floats, used in turn: a wave writes one only after the barrier of a block
-   * sum on the other, which every wave passes after reading this one's previous sums (no trailing barrier) */
-  __shared__ float red[4 * NW];
+  /* W: statistics in f64, for ragged rows past the 32 slots of the one-row-per-workgroup kernel, as the two-read
+   * kernel below takes them: f32 sums of squares are infinite there from an rms of about 6e16 on */
+  constexpr bool W = U && NV + NL > 32;
+  /* two block-sum buffers of 2 NW floats (W: doubles), used in turn: a wave writes one only after the barrier of a
+   * block sum on the other, which every wave passes after reading this one's previous sums (no trailing barrier) */
+  __shared__ float red[W ? 1 : 4 * NW];
+  __shared__ double redw[W ? 4 * NW : 1];
   int rb = 0;
 
   const int tid = threadIdx.x;
@@ -218,65 +266,86 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
       ++tl_row;
     }
 
-    /* one pass: sum and sum of squares */
-    float s = xe, q = xe * xe; /* 0 on lanes without an edge element */
+    /* the output is snake((x - lbase - vshift) A + beta); the LDS slots hold x, and so do the VGPR slots unless
+     * the centred pass below has subtracted lbase from them */
+    float vshift, lbase = 0.f, rstd;
+    if constexpr (W) {
+      double s = (double)xe, q = s * s;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      if (valid(k)) {
-        s += sum4(v[k]);
-        q = sumsq4(v[k], q);
-      }
-    }
-    /* LDS slots in groups of four: the scheduler would otherwise issue every
-     * slot's read at once and hold NL x 4 more VGPRs */
-    static_for<0, (NL + 3) / 4>([&](auto gc) {
-      constexpr int g = decltype(gc)::value;
-#pragma unroll
-      for (int m = 4 * g; m < (4 * g + 4 < NL ? 4 * g + 4 : NL); ++m) {
-        const nsr_float4 xl = lds_x[m * BLOCK + tid];
-        if (valid(NV + m)) {
-          s += sum4(xl);
-          q = sumsq4(xl, q);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    block_sum2<NW, false>(s, q, red + rb);
-    rb ^= 2 * NW;
-    const float mean = s * a.inv_t;
-    float var = __builtin_fmaf(-mean, mean, q * a.inv_t);
-    /* the VGPR slots hold x - vbase and the LDS slots x - lbase; (x - mean - c) A + beta = (x - vbase) A + Bc */
-    float vshift = mean, lbase = 0.f;
-    if (4.0f * mean * mean > var) {
-      /* second pass: centred sums; the VGPR slots keep x - mean (0 outside the row) */
-      const float de = edge_ok(rg) ? xe - mean : 0.f;
-      float s1 = de, s2 = de * de;
-#pragma unroll
-      for (int k = 0; k < NV; ++k) {
-        const nsr_float4 d = v[k] - mean;
-        v[k] = valid(k) ? d : zero4;
-        s1 += sum4(v[k]);
-        s2 = sumsq4(v[k], s2);
-      }
+      for (int k = 0; k < NV; ++k)
+        if (valid(k)) sums4_f64(v[k], s, q);
       static_for<0, (NL + 3) / 4>([&](auto gc) {
         constexpr int g = decltype(gc)::value;
 #pragma unroll
         for (int m = 4 * g; m < (4 * g + 4 < NL ? 4 * g + 4 : NL); ++m) {
-          nsr_float4 d = lds_x[m * BLOCK + tid] - mean;
-          d = valid(NV + m) ? d : zero4;
-          s1 += sum4(d);
-          s2 = sumsq4(d, s2);
+          const nsr_float4 xl = lds_x[m * BLOCK + tid];
+          if (valid(NV + m)) sums4_f64(xl, s, q);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
-      block_sum2<NW, false>(s1, s2, red + rb);
+      block_sum2_f64<NW>(s, q, redw + rb);
       rb ^= 2 * NW;
-      vshift = s1 * a.inv_t; /* f32 mean correction c */
-      lbase = mean;
-      var = __builtin_fmaf(-vshift, s1, s2) * a.inv_t;
+      row_moments(s, q, T, a.eps, lbase, vshift, rstd);
+    } else {
+      /* one pass: sum and sum of squares */
+      float s = xe, q = xe * xe; /* 0 on lanes without an edge element */
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        if (valid(k)) {
+          s += sum4(v[k]);
+          q = sumsq4(v[k], q);
+        }
+      }
+      /* LDS slots in groups of four: the scheduler would otherwise issue every
+       * slot's read at once and hold NL x 4 more VGPRs */
+      static_for<0, (NL + 3) / 4>([&](auto gc) {
+        constexpr int g = decltype(gc)::value;
+#pragma unroll
+        for (int m = 4 * g; m < (4 * g + 4 < NL ? 4 * g + 4 : NL); ++m) {
+          const nsr_float4 xl = lds_x[m * BLOCK + tid];
+          if (valid(NV + m)) {
+            s += sum4(xl);
+            q = sumsq4(xl, q);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      block_sum2<NW, false>(s, q, red + rb);
+      rb ^= 2 * NW;
+      const float mean = s * a.inv_t;
+      float var = __builtin_fmaf(-mean, mean, q * a.inv_t);
+      vshift = mean;
+      if (4.0f * mean * mean > var) {
+        /* second pass: centred sums; the VGPR slots keep x - mean (0 outside the row) */
+        const float de = edge_ok(rg) ? xe - mean : 0.f;
+        float s1 = de, s2 = de * de;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          const nsr_float4 d = v[k] - mean;
+          v[k] = valid(k) ? d : zero4;
+          s1 += sum4(v[k]);
+          s2 = sumsq4(v[k], s2);
+        }
+        static_for<0, (NL + 3) / 4>([&](auto gc) {
+          constexpr int g = decltype(gc)::value;
+#pragma unroll
+          for (int m = 4 * g; m < (4 * g + 4 < NL ? 4 * g + 4 : NL); ++m) {
+            nsr_float4 d = lds_x[m * BLOCK + tid] - mean;
+            d = valid(NV + m) ? d : zero4;
+            s1 += sum4(d);
+            s2 = sumsq4(d, s2);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        block_sum2<NW, false>(s1, s2, red + rb);
+        rb ^= 2 * NW;
+        vshift = s1 * a.inv_t; /* f32 mean correction c */
+        lbase = mean;
+        var = __builtin_fmaf(-vshift, s1, s2) * a.inv_t;
+      }
+      var = fmaxf(var, 0.0f);
+      rstd = __builtin_amdgcn_rsqf(var + a.eps); /* v_rsq_f32, about 1 ulp */
     }
-    var = fmaxf(var, 0.0f);
-    const float rstd = __builtin_amdgcn_rsqf(var + a.eps); /* v_rsq_f32, about 1 ulp */
     float gam, bet, alp;
     adain_params_cvt(pr, pdt, gam, bet, alp);
     const float A = (gam + 1.0f) * rstd;
@@ -319,7 +388,8 @@ NSR_DEV void adain_row(const nsr_adain_args& a, int pdt) {
       constexpr int k0 = decltype(gc)::value * SB;
       constexpr int k1 = k0 + SB < NV ? k0 + SB : NV;
 #pragma unroll
-      for (int k = k0; k < k1; ++k) buf_store4(orr, vo, (uint32_t)(k * BLOCK * 16), adain_snake4(v[k], A, Bc, sc));
+      for (int k = k0; k < k1; ++k)
+        buf_store4(orr, vo, (uint32_t)(k * BLOCK * 16), adain_snake4(W ? v[k] - lbase : v[k], A, Bc, sc));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = k0; k < k1; ++k) v[k] = vload(xn, k, vo, so + (uint32_t)(k * BLOCK * 16));
@@ -426,7 +496,8 @@ NSR_ADAIN_ROW(512, 39, 19)
  * access is split, and the edges cost one load and one store. Measured on MI355X, graph replays of one call, against
  * the kernels these rows took before (one workgroup per row; past T = 65,538 two reads of the row):
  * [8, 128, 115201] 210 against 554 us ([8, 128, 115200] on the aligned kernel: 185), [1, 128, 115201] 31 against 130,
- * [4, 128, 57601] 51 against 53.5, [8, 128, 28801] 47.5 against 52.0. */
+ * [4, 128, 57601] 51 against 53.5, [8, 128, 28801] 47.5 against 52.0. More than 32 slots sum in f64 (W): 0 to 1 us a
+ * call, [1, 128, 115201] 29.9 against 29.4 us with f32 sums, [8, 128, 115201] 194 against 195 (inputs rotated). */
 #define NSR_ADAIN_ROW_U(NV, NL)                                                             \
   extern "C" __global__ void __launch_bounds__(512)                                        \
       nsrk_adain_rowu_b512_v##NV##_l##NL(const nsr_adain_args a, const int pdt) {          \
@@ -1172,16 +1243,6 @@ NSR_DEV void row_sums64(const float* xr, int64_t T, double* red, double& s1, dou
     s2 += red[16 + w];
   }
   __syncthreads();
-}
-
-/* mean as an unevaluated f32 pair (hi + lo) and 1 / sqrt(var + eps) */
-NSR_DEV void row_moments(double s1, double s2, int64_t T, float eps, float& mhi, float& mlo, float& rstd) {
-  const double mean = s1 / (double)T;
-  double var = s2 / (double)T - mean * mean;
-  var = var > 0.0 ? var : 0.0;
-  mhi = (float)mean;
-  mlo = (float)(mean - (double)mhi);
-  rstd = 1.0f / sqrtf((float)var + eps);
 }
 
 /* Row statistics (mean, 1 / sqrt(var + eps)) of [n_rows][T] f32 into

@@ -14,10 +14,10 @@ from ._util import RTOL_F16, RTOL_F32, say
 pytestmark = pytest.mark.gpu
 
 
-def _closed_form(x, gam, bet, alp):
+def _closed_form(x, gam, bet, alp, eps=1e-5):
     x = x.double()
     m = x.mean(-1, keepdim=True)
-    y = (x - m) / torch.sqrt((x - m).square().mean(-1, keepdim=True) + 1e-5)
+    y = (x - m) / torch.sqrt((x - m).square().mean(-1, keepdim=True) + eps)
     y = y * (1.0 + gam.double()[:, :, None]) + bet.double()[:, :, None]
     al = alp.double()[None, :, None]
     return y + torch.sin(al * y).square() / (al + 1e-9)
@@ -59,3 +59,21 @@ def test_f32_rows(B, C, T):
 def test_f16_rows(B, C, T):
     say("adain ragged f16", B, C, T)
     _run(B, C, T, torch.float16, RTOL_F16, B + C + T)
+
+
+@pytest.mark.parametrize("T", [65543, 70001, 90002, 115201, 118790, 118797])
+def test_f32_statistics_range(T):
+    """Rows past the reach of the one-row-per-workgroup kernel keep statistics in f64: no overflow of the squares
+    at an rms where f32 sums of them are infinite (T x^2 > 3.4e38), none of a large mean's, and a variance below
+    the smallest normal f32 with eps = 0 (its f32 rounding, 2^-150 of 4e-40, moves 1 / sqrt(var) by 9e-7)."""
+    say("adain ragged f32, range of the statistics", T)
+    g = configs.rng(T)
+    rows = [(1.0, 0.0, 1e-5), (1e17, 0.0, 1e-5), (1e15, 3e17, 1e-5), (2e-20, 0.0, 0.0)]
+    for std, mean, eps in rows:
+        x = torch.from_numpy((g.standard_normal((1, 3, T)) * std + mean).astype(np.float32)).cuda()
+        gam, bet = (torch.from_numpy((g.standard_normal((1, 3)) * 0.1).astype(np.float32)).cuda() for _ in range(2))
+        alp = torch.ones(3, device="cuda")
+        ref = _closed_form(x, gam, bet, alp, eps)
+        out = abi.adain_snake(x, gam, bet, alp, eps=eps)
+        worst = float(((out.double() - ref).abs() / ref.abs().clamp_min(1.0)).max())
+        assert worst <= RTOL_F32, f"std {std} mean {mean}: {worst:.2e}"
