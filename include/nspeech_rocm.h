@@ -464,9 +464,10 @@ nsr_status nsr_adain_snake_conv1d_f32(const float* x, const void* gamma, const v
  * each x row) replaces the statistics pass over x when not NULL (the
  * previous stage's out_stats); out_stats, when not NULL, receives the same
  * pair for each row of out (after bias and residual), for the next stage's
- * AdaIN. The conv's epilogue produces them from
- * registers (per 32-column block count, mean and M2, merged per row by
- * Chan's pairwise formula) instead of a second read of out. Workspace:
+ * AdaIN. The conv's epilogue produces them from registers (mean and M2 per
+ * 32-column block, merged per row in f64) instead of a second read of out,
+ * which is left to the shapes of the fallback kernel and to rows whose blocks
+ * lose precision in f32 (see nsrk_conv_rowstats_merge). Workspace:
  * NSR_WS_IN_STATS when x_stats is NULL, NSR_WS_OUT_STATS when out_stats is
  * not NULL (0 bytes, workspace may be NULL, when neither). No counterpart
  * in the reference, whose ResBlock (src/kokoro/decoder.rs:1352-1380, GPU

@@ -37,6 +37,8 @@ typedef __attribute__((address_space(3))) nsr_float4 lds_f4;
 
 typedef _Float16 nsr_h8 __attribute__((ext_vector_type(8)));
 typedef float nsr_f32x16 __attribute__((ext_vector_type(16)));
+/* four f32 at any 4-byte aligned address (one 16-byte access) */
+typedef float cv_float4u __attribute__((ext_vector_type(4), aligned(4)));
 
 #define CV_TT 64            /* output columns per workgroup */
 #define CV_CO 128           /* output channels per workgroup */
@@ -1892,61 +1894,85 @@ extern "C" __global__ void __launch_bounds__(256) nsrk_conv1d_pack(const nsr_con
   a.wp[(co * a.K + k) * a.C_in + ci] = a.w[i];
 }
 
-/* Merge a row's (mean, M2) blocks (Chan, Golub and LeVeque's pairwise
- * update: n = na + nb, d = mb - ma, mean = ma + d nb / n,
- * M2 = M2a + M2b + d^2 na nb / n; block i holds min(32, T_out - 32 i)
- * columns) into the row's mean and 1 / sqrt(M2 / n + eps), the statistics
- * the fused AdaIN+Snake conv reads. One workgroup per row; each lane merges
- * blocks i = tid + 256 k in order (eight loads in flight at a time), then a
- * fixed tree over the lanes: the result does not depend on timing. */
-NSR_DEV void chan_merge(float& n, float& mean, float& m2, float nb, float mb, float m2b) {
-  const float nn = n + nb;
-  if (nb > 0.f) {
-    const float d = mb - mean;
-    const float f = nb / nn;
-    mean = __builtin_fmaf(d, f, mean);
-    m2 = m2 + m2b + d * d * n * f;
-    n = nn;
+/* Two f64 sums over the 256 lanes of the workgroup, in a fixed order. */
+NSR_DEV void sum2_256(double& a, double& b, double* red) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    a += __shfl_xor(a, off);
+    b += __shfl_xor(b, off);
   }
+  const int wid = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    red[wid] = a;
+    red[4 + wid] = b;
+  }
+  __syncthreads();
+  a = (red[0] + red[1]) + (red[2] + red[3]);
+  b = (red[4] + red[5]) + (red[6] + red[7]);
 }
 
+/* Merge a row's (mean, M2) blocks (block i holds n_i = min(32, T_out - 32 i) columns) into the row's mean and
+ * 1 / sqrt(var + eps), the statistics the fused AdaIN+Snake conv reads: with p the first block's mean,
+ * S1 = sum n_i (mean_i - p) and S2 = sum M2_i + n_i (mean_i - p)^2 in f64, mean = p + S1 / T and
+ * var = (S2 - S1^2 / T) / T. One workgroup per row, eight loads in flight per lane, sums in a fixed order: the
+ * result does not depend on timing.
+ * What the f32 blocks cannot give is taken from the row itself, read once more: a sum of squares that overflowed
+ * in a block, a variance too small for f32 squares (with eps as small), and, for rows whose statistics a pass
+ * over the output used to take (`reread`: rows that are not whole 16-byte vectors), mean^2 > 4 var, where the
+ * rounding of the block means shows: at |mean| = 1000 std 1 / sqrt(var) was off by 2e-6 at T = 2401, against
+ * 1e-7. */
 extern "C" __global__ void __launch_bounds__(256) nsrk_conv_rowstats_merge(const nsr_rowstats_args a) {
-  __shared__ float sn[256], sm[256], sq[256];
+  __shared__ double red[2][8];
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const nsr_float2* pr = (const nsr_float2*)a.part + row * a.nblk;
-  float n = 0.f, mean = 0.f, m2 = 0.f;
+  const double T = (double)a.T_out;
+  double p = (double)pr[0].x, s1 = 0.0, s2 = 0.0;
   for (int i0 = 0; i0 < a.nblk; i0 += 8 * 256) {
-    nsr_float2 p[8];
+    nsr_float2 b[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = pr[min(i0 + tid + 256 * u, a.nblk - 1)];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = i0 + tid + 256 * u;
-      p[u] = pr[min(i, a.nblk - 1)];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + tid + 256 * u;
-      const float nb = i < a.nblk ? (float)min(32, a.T_out - 32 * i) : 0.f;
-      chan_merge(n, mean, m2, nb, p[u].x, p[u].y);
+      if (i < a.nblk) {
+        const double d = (double)b[u].x - p, nd = (double)min(32, a.T_out - 32 * i) * d;
+        s1 += nd;
+        s2 += __builtin_fma(nd, d, (double)b[u].y);
+      }
     }
   }
-  sn[tid] = n;
-  sm[tid] = mean;
-  sq[tid] = m2;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (tid < w) {
-      float n0 = sn[tid], m0 = sm[tid], q0 = sq[tid];
-      chan_merge(n0, m0, q0, sn[tid + w], sm[tid + w], sq[tid + w]);
-      sn[tid] = n0;
-      sm[tid] = m0;
-      sq[tid] = q0;
+  sum2_256(s1, s2, red[0]);
+  double mean = p + s1 / T, var = (s2 - s1 * s1 / T) / T;
+  if (!(var < 1e300) || (float)var + a.eps < 1e-30f || (a.reread && mean * mean > 4.0 * var)) { /* workgroup-uniform */
+    const float* x = a.x + row * a.T_out;
+    p = fabs(mean) < 1e300 ? mean : 0.0;
+    s1 = 0.0;
+    s2 = 0.0;
+    auto add = [&](float v) {
+      const double d = (double)v - p;
+      s1 += d;
+      s2 = __builtin_fma(d, d, s2);
+    };
+    const int n4 = a.T_out >> 2;
+    for (int i0 = 0; i0 < n4; i0 += 4 * 256) {
+      nsr_float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = *(const cv_float4u*)(x + 4 * (int64_t)min(i0 + tid + 256 * u, n4 - 1));
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + tid + 256 * u < n4) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) add(v[u][e]);
+        }
     }
-    __syncthreads();
+    if (tid < (a.T_out & 3)) add(x[4 * n4 + tid]);
+    sum2_256(s1, s2, red[1]);
+    mean = p + s1 / T;
+    var = (s2 - s1 * s1 / T) / T;
   }
   if (tid == 0) {
-    const float var = fmaxf(sq[0] / fmaxf(sn[0], 1.f), 0.f);
-    a.stats[2 * row] = sm[0];
-    a.stats[2 * row + 1] = 1.0f / sqrtf(var + a.eps);
+    a.stats[2 * row] = (float)mean;
+    a.stats[2 * row + 1] = 1.0f / sqrtf((float)(var > 0.0 ? var : 0.0) + a.eps);
   }
 }

@@ -183,11 +183,12 @@ typedef struct nsr_conv_args {
 
 typedef struct nsr_rowstats_args {
   const float* part;       /* [rows][nblk][2] (mean, M2) of 32-column blocks */
+  const float* x;          /* [rows][T_out], the rows themselves */
   float* stats;            /* [rows][2] mean, 1 / sqrt(var + eps) */
   int32_t nblk;
   int32_t T_out;           /* block i holds min(32, T_out - 32 i) columns */
   float eps;
-  int32_t pad_;
+  int32_t reread;          /* 1: rows with mean^2 > 4 var are read again (see nsrk_conv_rowstats_merge) */
 } nsr_rowstats_args;
 
 typedef struct nsr_conv_pack_args {

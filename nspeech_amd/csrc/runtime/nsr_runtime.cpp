@@ -1609,8 +1609,8 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
 }
 
 // Launch a conv and leave the per-(b, co) statistics of its output in row_stats ([B*C_out][2]: mean,
-// 1 / sqrt(var + eps)): the aligned-row kernels emit per-32-column (mean, M2) blocks from their epilogue into
-// `part` (the caller's workspace, [B*C_out][ceil(T_out / 32)][2] f32) and a merge kernel combines them; the
+// 1 / sqrt(var + eps)): the record and one-launch kernels emit per-32-column (mean, M2) blocks from their epilogue
+// into `part` (the caller's workspace, [B*C_out][ceil(T_out / 32)][2] f32) and a merge kernel combines them; the
 // fallback kernel's output is re-read by the row statistics kernel instead.
 static nsr_status conv_launch_stats(bool fused, nsr_conv_args& a, float eps, float* row_stats, float* part,
                                     char* records, nsr_stream_t stream, const char* what) {
@@ -1623,6 +1623,8 @@ static nsr_status conv_launch_stats(bool fused, nsr_conv_args& a, float eps, flo
     nsr_rowstats_args m;
     std::memset(&m, 0, sizeof(m));
     m.part = part;
+    m.x = a.out;
+    m.reread = a.T_out % 4 != 0 || !aligned(a.out, 16);
     m.stats = row_stats;
     m.nblk = (int32_t)nblk;
     m.T_out = a.T_out;

@@ -1,8 +1,8 @@
 """Row statistics handed along the Kokoro ResBlock chain
 (nsr_conv1d_f16w_packed_stats, nsr_adain_snake_conv1d_chain_f32): the
-conv's epilogue emits (count, mean, M2) per row and 32-column block, a
-merge kernel combines them (Chan's pairwise formula), and the next fused
-AdaIN+Snake conv takes them instead of re-reading its input.
+conv's epilogue emits (mean, M2) per row and 32-column block, a merge
+kernel combines them in f64, and the next fused AdaIN+Snake conv takes them
+instead of re-reading its input.
 
 Checks: the output itself is bit-identical to the conv without statistics;
 the statistics match the float64 mean and 1 / sqrt(var + eps) of that

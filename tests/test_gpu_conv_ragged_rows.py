@@ -160,3 +160,25 @@ def test_resident_weight_kernel(C, T, K, dil, pad, res):
     spread = torch.sqrt(d.var(-1, unbiased=False) + 1e-5)
     assert bool(((st[:, 0].double() - d.mean(-1)).abs() <= 1e-5 * torch.maximum(d.mean(-1).abs(), spread)).all())
     assert bool(((st[:, 1].double() * spread - 1.0).abs() <= 1e-5).all())
+
+
+@pytest.mark.parametrize("C_out,T,K", [(128, 31, 3), (128, 333, 7), (128, 2401, 3), (96, 2402, 11), (128, 19201, 7)])
+def test_row_statistics_of_ragged_rows(C_out, T, K):
+    """The statistics handed along, for outputs of |mean| up to 1000 std and up to 1e19 (the residual sets both):
+    the mean within its f32 rounding and that of block means up to 2 std, 2^-24 |mean| + 2^-22 std; 1 / sqrt(var)
+    within 10 u (u = 2^-24: nine roundings of a block's sum of squares, halved by the root, then those of the sum
+    with eps, the root and the division)."""
+    g = configs.rng(T + K)
+    x = torch.from_numpy(g.standard_normal((2, 128, T)).astype(np.float32)).cuda()
+    w = torch.from_numpy((g.standard_normal((C_out, 128, K)) / np.sqrt(128 * K)).astype(np.float16)).cuda()
+    wp = abi.conv1d_pack_f16(w)
+    n = torch.from_numpy(g.standard_normal((2, C_out, T)).astype(np.float32)).cuda()
+    for std, mean in ((1.0, 0.0), (1.0, 3.0), (1.0, 30.0), (1.0, -1000.0), (1e17, 0.0), (1e19, 0.0), (1e15, 3e17)):
+        say("conv statistics of ragged rows", C_out, T, K, std, mean)
+        for records in (True, False):
+            o, st = abi.conv1d_f16w_packed_stats(x, wp, None, n * std + mean, padding=(K - 1) // 2, records=records)
+            d, st = o.double().view(2 * C_out, T), st.double()
+            m, sd = d.mean(-1), torch.sqrt(d.var(-1, unbiased=False) + 1e-5)
+            em = ((st[:, 0] - m).abs() / (2.0 ** -24 * m.abs() + 2.0 ** -22 * sd)).max()
+            er = (st[:, 1] * sd - 1.0).abs().max() / (10 * 2.0 ** -24)
+            assert em <= 1.0 and er <= 1.0, f"std {std} mean {mean} records={records}: {em:.2f}, {er:.2f} of the bars"
