@@ -789,11 +789,15 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
       kid = ids[nv == 39 ? 19 : nv / 2 - 1];
       lds = (unsigned)(nl * 512 * 16);
     }
-    if (lds + 1024 <= (unsigned)dm->max_lds) block = 512;
     // the kernel masks only its last four slots at the row end
-    if (block && (int64_t)(nv + nl - 4) * 512 > nmin)
+    if ((int64_t)(nv + nl - 4) * 512 > nmin)
       return fail(NSR_ERR_HIP, "adain_snake: internal error: row kernel slots do not fit T=%lld", (long long)T);
-    persistent = true;
+    if (lds + 1024 <= (unsigned)dm->max_lds) {
+      block = 512;
+      persistent = true;
+    } else {
+      lds = 0;  // no room for the LDS slots: the kernels below, one workgroup per row
+    }
   }
   if (!is_aligned && !block) {
     // Unaligned rows: interior chunks 1..nch-2 resident in VGPRs, edges by element.
