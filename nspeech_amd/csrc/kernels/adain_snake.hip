@@ -491,8 +491,8 @@ NSR_ADAIN_ROW(512, 37, 19)
 NSR_ADAIN_ROW(512, 38, 19)
 NSR_ADAIN_ROW(512, 39, 19)
 
-/* Rows past T = 8192 that are not a multiple of 4 long. VGPR slots up to 19, 19 LDS slots and an even number of
- * VGPR slots beyond. What bounds it is what bounds the aligned rows; the chunks stay on the 16-byte grid, so no
+/* Rows that are not a multiple of 4 long, where the host's rule takes them (ragged_row_kernel). VGPR slots up to
+ * 19, 19 LDS slots and an even number of VGPR slots beyond. What bounds it is what bounds the aligned rows; the chunks stay on the 16-byte grid, so no
  * access is split, and the edges cost one load and one store. Measured on MI355X, graph replays of one call, against
  * the kernels these rows took before (one workgroup per row; past T = 65,538 two reads of the row):
  * [8, 128, 115201] 210 against 554 us ([8, 128, 115200] on the aligned kernel: 185), [1, 128, 115201] 31 against 130,
@@ -506,7 +506,6 @@ NSR_ADAIN_ROW(512, 39, 19)
 NSR_ADAIN_ROW_U(6, 0)
 NSR_ADAIN_ROW_U(8, 0)
 NSR_ADAIN_ROW_U(10, 0)
-NSR_ADAIN_ROW_U(12, 0)
 NSR_ADAIN_ROW_U(16, 0)
 NSR_ADAIN_ROW_U(20, 0)
 NSR_ADAIN_ROW_U(2, 19)

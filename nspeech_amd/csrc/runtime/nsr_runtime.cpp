@@ -665,6 +665,29 @@ nsr_status nsr_attention_decode_f16(const void* q, const void* k, const void* v,
 
 // -------------------------------------------------------- AdaIN + Snake --
 
+// Rows of T % 4 != 0 elements: the persistent row kernel, or the kernel of one workgroup per row (rows of up to 32
+// slots of 512 16-byte chunks; the row kernel alone past them, where the other choice reads each row twice).
+// Measured on MI355X, row kernel / other, us per graph replay, inputs rotated past the caches (in brackets: one input
+// again and again, where the row kernel gains from the loads it caches):
+//   up to 8197 elements the other kernel has 256 lanes: [1, 1024, 8193] (14.8 / 12.0)
+//   4.3 slots, 256, 1024, 2048 rows: 5.3 / 6.0, 15.4 / 16.7, 27.3 / 29.9
+//   5.9 slots, 256, 1024, 1280 rows: 6.3 / 6.7, 20.8 / 20.7, 28.2 / 25.4
+//   8.0 slots, 128, 512, 1024 rows: 5.9 / 6.2, 14.0 / 13.0, 27.0 / 27.1
+//   9.4 slots, 128, 512, 1024 rows: 6.5 / 6.7, 16.3 / 15.1, 32.8 / 31.5; 11.7 slots: 7.5 / 7.4, 20.4 / 18.8, 40.6 / 39.3
+//   14 slots, 128, 400, 1024 rows: 8.6 / 8.5, 21.4 / 19.6, 48.5 / 49.8 (8.3 / 9.2, -, 43.9 / 48.2)
+//   19.5 slots, 128, 256, 1024, 2048 rows: 11.2 / 10.8, 18.6 / 17.4, 70.6 / 68.8, 135 / 127
+//     (8.9 / 11.6, 17.3 / 16.2, 52.5 / 66.5, 133 / 126)
+//   28 slots, 128, 256, 1024, 2048 rows: 15.0 / 15.0, 25.9 / 25.0, 98.8 / 100.5, 190 / 190
+//     (11.8 / 16.2, 24.6 / 23.0, 74.8 / 95.7, 189 / 188)
+//   34 slots, 128, 1024 rows: 18.3 / 77.3, 117 / 329
+static bool ragged_row_kernel(int64_t n_rows, int64_t T, int n_cu) {
+  const int64_t nch = (T + 6) / 4 - 2, slots = (nch + 511) / 512;
+  if (T % 4 == 0 || nch <= 256 * 8 || slots > 39 + 19) return false;
+  if (slots > 32 || slots <= 5) return true;
+  if (slots <= 12) return n_rows <= (slots <= 6 ? 4 * n_cu : slots <= 10 ? n_cu : 0);
+  return 2 * n_rows <= n_cu || (n_rows >= 2 * n_cu && (slots <= 19 || n_rows <= 5 * n_cu));
+}
+
 nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* beta, const void* alpha,
                                nsr_dtype param_dtype, int64_t gamma_bstride, int64_t beta_bstride,
                                float* out, int64_t B, int64_t C, int64_t T, float eps,
@@ -756,19 +779,16 @@ nsr_status nsr_adain_snake_f32(const float* x, const void* gamma, const void* be
     const int ns = nv + nl;
     if (block && (int64_t)(ns - std::min(ns, 4)) * block > nch)
       return fail(NSR_ERR_HIP, "adain_snake: internal error: row kernel slots do not fit T=%lld", (long long)T);
-  } else if (aligned(x, 16) && aligned(out, 16) && T > 8 * 1024 && (T + 6) / 4 - 2 <= 512 * (39 + 19)) {
-    // Rows of T % 4 != 0 elements past the 256-lane kernels: the row kernel over the interior chunks of the 16-byte
-    // grid, edges by element (ceil(T / 4) - 2 to (T + 6) / 4 - 2 interior chunks, by the row's start). Against the
-    // one-row-per-workgroup kernel below and the two-read kernel past its 32 slots, us per graph
-    // replay: [8, 128, 12001] 24.1 / 24.0, [8, 128, 28801] 47.5 / 52.0, [4, 128, 57601] 51.0 / 53.5,
-    // [8, 128, 115201] 210 / 554, [1, 128, 115201] 31 / 130.
+  } else if (aligned(x, 16) && aligned(out, 16) && ragged_row_kernel(n_rows, T, dm->n_cu)) {
+    // Rows of T % 4 != 0 elements: the row kernel over the interior chunks of the 16-byte grid, edges by element
+    // (ceil(T / 4) - 2 to (T + 6) / 4 - 2 interior chunks, by the row's start).
     const int64_t nch = (T + 6) / 4 - 2, nmin = (T + 3) / 4 - 2;
     int nv = 0, nl = 0;
     if (nch <= 512 * 19) {
-      static const int opts[] = {6, 8, 10, 12, 16, 20};
-      static const KId ids[] = {K_nsrk_adain_rowu_b512_v6_l0,  K_nsrk_adain_rowu_b512_v8_l0,  K_nsrk_adain_rowu_b512_v10_l0,
-                                K_nsrk_adain_rowu_b512_v12_l0, K_nsrk_adain_rowu_b512_v16_l0, K_nsrk_adain_rowu_b512_v20_l0};
-      for (int i = 0; i < 6 && !nv; ++i)
+      static const int opts[] = {6, 8, 10, 16, 20};
+      static const KId ids[] = {K_nsrk_adain_rowu_b512_v6_l0, K_nsrk_adain_rowu_b512_v8_l0, K_nsrk_adain_rowu_b512_v10_l0,
+                                K_nsrk_adain_rowu_b512_v16_l0, K_nsrk_adain_rowu_b512_v20_l0};
+      for (int i = 0; i < 5 && !nv; ++i)
         if (512LL * opts[i] >= nch) {
           nv = opts[i];
           kid = ids[i];

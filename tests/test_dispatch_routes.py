@@ -102,3 +102,14 @@ def test_adain_rows_without_room_for_lds_slots(routes):
         k, gx, _, _, block, lds = log[0]
         assert "_l19" not in k and lds == 0, log
         _check_adain(r, T, off, k, gx, block, lds)
+
+
+@pytest.mark.parametrize("rows,T,row_kernel", [
+    (1024, 8193, False), (1024, 8201, True), (2048, 9001, True), (1024, 12001, True), (1280, 12001, False),
+    (256, 14401, True), (512, 14401, False), (128, 19201, True), (1024, 19201, False), (128, 24001, False),
+    (128, 28801, True), (400, 28801, False), (1024, 28801, True), (3000, 28801, True), (128, 48001, True),
+    (256, 48001, False), (1024, 57601, True), (2048, 40001, False), (256, 70001, True), (3000, 115201, True)])
+def test_adain_ragged_rows_take_the_faster_kernel(routes, rows, T, row_kernel):
+    """Each side of the rule's lines (measured: see the rule), where the other kernel was slower or no faster."""
+    (st, log), = routes([_adain(rows, T)])
+    assert st == 0 and log[0][0].startswith("nsrk_adain_rowu_") == row_kernel, log
