@@ -1476,6 +1476,72 @@ const KId kConvNp[2][3] = {
     {K_nsrk_conv1d_f16x2_np9, K_nsrk_conv1d_f16x2_np12, K_nsrk_conv1d_f16x2_np16},
     {K_nsrk_conv1d_adain_snake_f16x2_np9, K_nsrk_conv1d_adain_snake_f16x2_np12, K_nsrk_conv1d_adain_snake_f16x2_np16}};
 
+// Every row of a conv's tensors on whole 16-byte vectors: its output (and residual), and its input as well.
+bool conv_out16(const nsr_conv_args& a) {
+  return a.T_out % 4 == 0 && aligned(a.out, 16) && (!a.residual || aligned(a.residual, 16));
+}
+bool conv_rows16(const nsr_conv_args& a) { return conv_out16(a) && a.T_in % 4 == 0 && aligned(a.x, 16); }
+
+// What the rules below measure a shape by.
+struct ConvSize {
+  int64_t n_ch, n_co;  // 128-channel blocks of the input and the output
+  int64_t tiles;       // 128 x 64 tiles of the one-launch kernels, one at a time per CU
+  bool wide, full;     // channels enough to fill the kernels' 128 x 128 products: in part, wholly
+  bool two;            // the fallback kernel runs two workgroups per CU (plain input, short halo)
+};
+ConvSize conv_size(const nsr_conv_args& a, bool fused) {
+  ConvSize s;
+  s.n_ch = (a.C_in + kCvCI - 1) / kCvCI;
+  s.n_co = (a.C_out + kCvCO - 1) / kCvCO;
+  s.tiles = (int64_t)cdiv_u(a.T_out, kCvTT) * s.n_co * a.B;
+  s.wide = (int64_t)a.C_in * a.C_out >= 64 * 128;
+  s.full = a.C_in > 96 && a.C_out > 96;
+  s.two = !fused && kCvTT + (int64_t)(a.K - 1) * a.dilation <= 72;
+  return s;
+}
+
+// Rows that are not whole 16-byte vectors: is the fallback kernel faster than the producer / consumer kernels?
+// Those fill a pipeline of two tiles first and multiply whole 128-channel blocks, so they pay with several tiles per
+// CU, with several input blocks, and where the channels fill a block; the fallback kernel stops at C_in, runs two
+// workgroups per CU on plain inputs with a short halo, and needs a statistics pass of its own. MI355X, us per
+// graph replay, fallback / the other, dilation 1 (measured over 13 channel pairs, 6 kernel sizes, dilation 1 and 5 and 12 tile counts):
+//   fused, statistics out: 128 -> 128 K = 3, 16 / 64 / 256 tiles 19.2 / 21.9, 22.1 / 22.3, 26.8 / 24.1; K = 5, 64 tiles
+//     25.0 / 28.1, 512 tiles 46.7 / 31.2; 64 -> 64 K = 3, 64 tiles 16.4 / 21.7, 1024 tiles 50.8 / 33.7;
+//     256 -> 256 K = 3, 64 tiles 32.2 / 25.6
+//   fused: 128 -> 128 K = 3, 256 tiles 17.6 / 19.5; 64 -> 64 K = 5, 512 tiles 26.4 / 24.5
+//   plain: 128 -> 128 K = 3, 16 tiles 16.1 / 15.3; K = 5, 64 tiles 19.3 / 22.6, 512 tiles 28.4 / 26.2;
+//     64 -> 64 K = 5, 1024 tiles 31.4 / 38.8; 512 -> 32 K = 5, 64 tiles 39.0 / 34.6, 512 tiles 56.3 / 65.3
+// Over all of them the choice costs 0.3% on average against the better one, at most 27% (narrow channels, 5 to 9 us).
+// Where only the input's rows are ragged (an even K, padding on one side) the fallback kernel stores 16-byte vectors and
+// is about 14% faster than that: 128 -> 128 K = 2, 64 tiles plain 12.8 / 14.5, fused 12.3 / 17.7; K = 4, 1024 tiles plain
+// 39.0 / 39.0, fused 58.6 / 42.7; 256 -> 256 K = 2, 16 tiles fused 17.5 / 20.8, 512 tiles plain 24.0 / 28.0.
+bool conv_fallback_faster(const nsr_conv_args& a, bool fused, int64_t n_cu) {
+  const ConvSize s = conv_size(a, fused);
+  if (conv_out16(a)) {
+    if (s.n_ch > 1)
+      return s.tiles > n_cu ? s.two : fused && a.K <= 2 && !(a.row_part && a.C_out > 64 && 4 * s.tiles >= n_cu);
+    return !(s.tiles > (s.two ? 3 : 1) * n_cu && a.C_in >= 64 && (a.K <= 3 || (s.two ? s.full : s.wide)));
+  }
+  if (s.n_ch > 1) return s.two && s.tiles > n_cu && (a.C_out <= 64 || s.n_ch >= 4);
+  if (s.tiles > n_cu) {
+    if (a.K <= 3 && !s.two) return false;
+    return !(s.two && a.K > 3 ? s.full : s.wide || (a.C_in >= 64 && s.tiles > 3 * n_cu));
+  }
+  if (a.K > 3) return true;
+  if (fused) return !(a.row_part && (s.full ? 4 * s.tiles >= n_cu : s.wide && a.C_out > 64 && 2 * s.tiles >= n_cu));
+  return !(s.n_co == 1 && a.C_out > 96 && a.C_in >= 64);
+}
+
+// Such rows with K >= 7 (rows of whole vectors: always): is the record path faster than both? Its records hold whole
+// 128-channel blocks, written and read whatever C_in is. Fallback / records, as above: 128 -> 128 K = 7, 64 tiles fused
+// 21.3 / 15.1, plain 22.0 / 16.0, 1024 tiles fused 86.2 / 54.6, plain 59.3 / 56.3; 64 -> 64 K = 7, 64 tiles plain
+// 16.8 / 15.2, 512 tiles 20.8 / 28.2 (fused 30.2 / 28.0); 32 -> 32 K = 7, 64 tiles fused 13.3 / 14.5, plain 14.2 / 15.0.
+bool conv_records_faster_ragged(const nsr_conv_args& a, bool fused, int64_t n_cu) {
+  const ConvSize s = conv_size(a, fused);
+  if (s.two) return s.full || (s.wide && s.tiles <= n_cu) || (a.C_in >= 64 && 2 * s.tiles <= n_cu);
+  return s.wide || (a.C_in >= 64 && (2 * s.tiles <= n_cu || s.tiles > 3 * n_cu)) || 16 * s.tiles <= n_cu;
+}
+
 nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const char* what, bool* emitted = nullptr) {
   DeviceModule* dm = nullptr;
   nsr_status st = current_module(&dm);
@@ -1485,8 +1551,7 @@ nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const 
   if (TL > kCvMaxTL || lds > dm->max_lds)
     return fail(NSR_ERR_UNSUPPORTED, "%s: (K - 1) * dilation = %lld needs %lld bytes of LDS, device allows %d", what,
                 (long long)((a.K - 1) * (int64_t)a.dilation), (long long)lds, dm->max_lds);
-  // 16-byte epilogue stores when every output (and residual) row starts 16-byte aligned
-  a.pad_ = (a.T_out % 4 == 0 && aligned(a.out, 16) && (!a.residual || aligned(a.residual, 16))) ? 1 : 0;
+  a.pad_ = conv_out16(a) ? 1 : 0;  // the fallback kernel's 16-byte epilogue stores
   void* params[] = {&a};
   // persistent workgroups: as many as fit at once (two per CU when the LDS allows), each walking tiles
   const int64_t tiles = (int64_t)cdiv_u(a.T_out, kCvTT) * cdiv_u(a.C_out, kCvCO) * a.B;
@@ -1499,7 +1564,8 @@ nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const 
   // both kernels below form 32-bit offsets of whole 128-channel blocks and 64-column tiles, those past the
   // output included, and leave dropping them to the range check: they must not wrap
   const bool fits32 = 4 * (int64_t)cdiv_u(a.C_out, kCvCO) * kCvCO * ((int64_t)a.T_out + kCvTT) <= kConvMaxSlabBytes;
-  if (a.C_in <= kCvCI && a.C_out <= kCvCO && a.K <= 3 && win <= 128 && lds_rw <= dm->max_lds && a.T_in > 0 && fits32) {
+  const bool pipelined = win <= 128 && a.T_in > 0 && fits32 && (conv_rows16(a) || !conv_fallback_faster(a, fused, dm->n_cu));
+  if (pipelined && a.C_in <= kCvCI && a.C_out <= kCvCO && a.K <= 3 && lds_rw <= dm->max_lds) {
     const int64_t groups = std::min<int64_t>(tiles, (int64_t)dm->n_cu);
     if (emitted) *emitted = a.row_part != nullptr;
     return launch(kConvRw[fused][a.residual != nullptr][a.row_part != nullptr][win <= 96 ? 0 : 1], (unsigned)groups,
@@ -1508,7 +1574,7 @@ nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const 
   // any K, C_in in chunks and C_out in blocks of 128: weights streamed one tap ahead
   // through two LDS slots, one 512-lane workgroup per CU (producer and consumer waves)
   const int64_t lds_pc = (2 * TL + 2 * kCvCO) * kCvS * 2 + 4 * (int64_t)a.C_out; /* + the bias as f32 */
-  if (win <= 128 && lds_pc <= dm->max_lds && a.T_in > 0 && fits32) {
+  if (pipelined && lds_pc <= dm->max_lds) {
     const int64_t groups = std::min<int64_t>(tiles, (int64_t)dm->n_cu);
     if (emitted) *emitted = a.row_part != nullptr;
     return launch(kConvPc[fused][a.residual != nullptr][a.row_part != nullptr][win <= 96 ? 0 : 1], (unsigned)groups,
@@ -1572,7 +1638,8 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   // one-launch kernel transforms its input once per output block and the records win from K = 3:
   // [8, 256, 9600] 571 against 639 us, [4, 256, 3200] 147 against 173 us, [1, 256, 3200] 87 against 110 us.
   const bool blocks1 = a.C_in <= kCvCI && a.C_out <= kCvCO;
-  if (!records || a.K < (blocks1 ? 7 : 3) || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0)
+  if (!records || a.K < (blocks1 ? 7 : 3) || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0 ||
+      (a.K >= 7 && !conv_out16(a) && !conv_records_faster_ragged(a, fused, dm->n_cu)))
     return conv_launch(fused, a, stream, what, emitted);
   const int64_t Tp = (int64_t)a.T_in + 2 * a.padding;
   const int64_t n_ch = (a.C_in + 127) / 128, n_co = (a.C_out + 127) / 128;

@@ -20,7 +20,8 @@ void fake_hip_set(int lds, int cus, int occupancy) {
   g_occupancy = occupancy;
 }
 
-// The launches since the last call: "name gx gy gz block lds" lines.
+// The launches since the last call: "name gx gy gz block lds n" lines, n the tile argument of the conv's record kernels
+// (their fourth), 0 for others.
 const char* fake_hip_take_log(void) {
   g_out.swap(g_log);
   g_log.clear();
@@ -59,9 +60,11 @@ hipError_t hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(int* n, hipFunctio
 }
 
 hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned,
-                                 unsigned, unsigned lds, hipStream_t, void**, void**) {
+                                 unsigned, unsigned lds, hipStream_t, void** params, void**) {
+  const char* name = (const char*)f;
+  const bool tiles = !std::strncmp(name, "nsrk_conv1d_pr_", 15) || !std::strncmp(name, "nsrk_conv1d_ps", 14);
   char line[256];
-  std::snprintf(line, sizeof(line), "%s %u %u %u %u %u\n", (const char*)f, gx, gy, gz, bx, lds);
+  std::snprintf(line, sizeof(line), "%s %u %u %u %u %u %d\n", name, gx, gy, gz, bx, lds, tiles ? *(const int*)params[3] : 0);
   g_log += line;
   return hipSuccess;
 }

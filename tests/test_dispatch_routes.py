@@ -1,6 +1,6 @@
 """Which kernels a call launches, without a GPU: the built library is loaded over a recording HIP runtime
 (tests/host/fake_hip.cpp) in a process of its own, its entry points are called with addresses that nothing reads,
-and the launches (kernel, grid, block, LDS bytes) are checked against what each kernel assumes."""
+and the launches (kernel, grid, block, LDS bytes, tile argument) are checked against what each kernel assumes."""
 import json
 import re
 import subprocess
@@ -33,7 +33,7 @@ json.dump(out, sys.stdout)
 
 @pytest.fixture(scope="module")
 def routes(tmp_path_factory):
-    """routes(calls, lds, cus) -> [(status, [(kernel, gx, gy, gz, block, lds), ...])], one per call."""
+    """routes(calls, lds, cus) -> [(status, [(kernel, gx, gy, gz, block, lds, n), ...])], one per call."""
     if not LIB.exists():
         pytest.fail(f"{LIB} is not built: run `python -m nspeech_amd.build`")
     so = tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so"
@@ -89,7 +89,7 @@ def test_adain_launches_cover_every_row(routes):
     cases = [(r, T, off) for r in ROWS for T in _lengths() for off in (0, 4)]
     for (r, T, off), (st, log) in zip(cases, routes([_adain(*c) for c in cases])):
         assert st == 0 and len(log) == 1, (r, T, off, st, log)
-        k, gx, gy, gz, block, lds = log[0]
+        k, gx, gy, gz, block, lds, _ = log[0]
         assert (gy, gz) == (1, 1)
         _check_adain(r, T, off, k, gx, block, lds)
 
@@ -99,7 +99,7 @@ def test_adain_rows_without_room_for_lds_slots(routes):
     cases = [(3000, T, 0) for T in (40001, 50002, 65537, 70001, 115203, 40000, 115200)]
     for (r, T, off), (st, log) in zip(cases, routes([_adain(*c) for c in cases], lds=100000)):
         assert st == 0 and len(log) == 1, (r, T, st, log)
-        k, gx, _, _, block, lds = log[0]
+        k, gx, _, _, block, lds, _ = log[0]
         assert "_l19" not in k and lds == 0, log
         _check_adain(r, T, off, k, gx, block, lds)
 
@@ -113,3 +113,94 @@ def test_adain_ragged_rows_take_the_faster_kernel(routes, rows, T, row_kernel):
     """Each side of the rule's lines (measured: see the rule), where the other kernel was slower or no faster."""
     (st, log), = routes([_adain(rows, T)])
     assert st == 0 and log[0][0].startswith("nsrk_adain_rowu_") == row_kernel, log
+
+
+def _conv(mode, C_in, C_out, B, T, K, dil, records, res=False, off=0, pad=None):
+    """mode "stats" / "fused": adain_snake_conv1d_chain with / without statistics out; "plain": conv1d_f32io."""
+    pad = (K - 1) * dil // 2 if pad is None else pad
+    T_out = T + 2 * pad - dil * (K - 1)
+    x, out, r = [("p", (v << 40) + off) for v in (1, 2, 3)]
+    big, ws = 1 << 46, ("p", 1 << 47)
+    if mode == "plain":
+        need = -(-2 * C_in * C_out * K // 256) * 256
+        return ["nsr_conv1d_f32io", [x, ("p", 256), ("p", 0), out, ("l", B), ("l", C_in), ("l", C_out), ("l", T), ("l", K),
+                                     ("l", 1), ("l", pad), ("l", dil), ws, ("l", big if records else need), ("p", 0)]]
+    need = -(-8 * B * C_out * -(-T_out // 32) // 256) * 256 if mode == "stats" else 0
+    a = [("p", 256)] * 3
+    return ["nsr_adain_snake_conv1d_chain_f32",
+            [x, ("p", 256), *a, ("i", NSR_F32), ("l", 0), ("l", 0), ("p", 256), ("p", 0), r if res else ("p", 0), out,
+             ("p", 256 if mode == "stats" else 0), ("l", B), ("l", C_in), ("l", C_out), ("l", T), ("l", K), ("l", pad),
+             ("l", dil), ("f", 1e-5), ws, ("l", big if records else need), ("p", 0)]]
+
+
+def _family(log):
+    names = [l[0] for l in log if l[0].startswith("nsrk_conv1d_") and l[0] != "nsrk_conv1d_pack"]
+    kinds = {"records" if re.search(r"_p[rs]\d?_", n) else "one launch" if re.search(r"_(rw|pc)_", n) else "fallback"
+             for n in names}
+    assert len(kinds) == 1, log
+    return kinds.pop()
+
+
+@pytest.mark.parametrize("mode,C_in,C_out,B,T,K,dil,records,family", [
+    # rows of T % 4 != 0, one dilation, where the kernels before or beside the choice were 10% slower or more
+    ("plain", 16, 16, 4, 401, 3, 1, True, "fallback"), ("fused", 16, 16, 4, 2401, 2, 5, False, "fallback"),
+    ("stats", 64, 64, 4, 1021, 3, 1, False, "fallback"), ("stats", 64, 64, 4, 16381, 3, 1, False, "one launch"),
+    ("stats", 128, 128, 1, 1021, 3, 1, False, "fallback"), ("stats", 128, 128, 4, 4093, 3, 1, False, "one launch"),
+    ("fused", 128, 128, 4, 4093, 3, 1, False, "fallback"), ("stats", 128, 128, 1, 19201, 3, 1, True, "one launch"),
+    ("stats", 128, 128, 4, 1021, 5, 1, True, "fallback"), ("stats", 128, 128, 4, 8189, 5, 1, True, "one launch"),
+    ("plain", 128, 128, 1, 1021, 3, 1, False, "one launch"), ("plain", 128, 128, 4, 1021, 5, 1, False, "fallback"),
+    ("plain", 64, 64, 4, 16381, 5, 1, False, "fallback"), ("plain", 256, 256, 1, 401, 7, 1, False, "one launch"),
+    ("plain", 512, 32, 4, 8189, 5, 1, False, "fallback"), ("stats", 256, 256, 4, 509, 2, 1, False, "one launch"),
+    ("plain", 128, 128, 1, 2401, 7, 1, True, "records"), ("stats", 128, 128, 1, 19201, 7, 5, True, "records"),
+    ("stats", 128, 128, 4, 57601, 11, 5, True, "records"), ("plain", 64, 64, 4, 8189, 7, 1, True, "fallback"),
+    ("plain", 32, 32, 4, 8189, 7, 1, True, "fallback"), ("plain", 64, 64, 4, 1021, 7, 1, True, "records"),
+    # ragged inputs of an even K, outputs of whole vectors
+    ("plain", 128, 128, 4, 1025, 2, 1, True, "fallback"), ("fused", 256, 256, 1, 1021, 2, 1, True, "fallback"),
+    ("fused", 128, 128, 4, 16381, 2, 1, True, "one launch"), ("plain", 256, 256, 4, 4097, 2, 1, True, "fallback"),
+    # rows of whole vectors keep the kernels they had
+    ("plain", 16, 16, 4, 400, 3, 1, True, "one launch"), ("plain", 32, 32, 4, 8188, 7, 1, True, "records"),
+    ("stats", 128, 128, 8, 115200, 3, 5, True, "one launch"), ("stats", 256, 256, 1, 3200, 11, 3, True, "records")])
+def test_conv_takes_the_faster_kernels(routes, mode, C_in, C_out, B, T, K, dil, records, family):
+    (st, log), = routes([_conv(mode, C_in, C_out, B, T, K, dil, records)])
+    assert st == 0 and _family(log) == family, log
+
+
+def _record_columns(log, B, T_out, C_out):
+    """The 64-column tiles of the output that a record call's launches write, as (channel block of 64, batch, tile)."""
+    n64, n128, seen = -(-T_out // 64), -(-T_out // 128), []
+    for k, gx, gy, gz, block, lds, n in log:
+        if k.startswith("nsrk_conv1d_pr_"):
+            n_co = -(-C_out // 128)
+            assert (gy, gz, block) == (1, 1, 512) and 1 <= gx <= CUS
+            for tile in range(n):  # channel block fastest, then columns, then batch
+                col, cb = divmod(tile, n_co)
+                b, t = divmod(col, n128)
+                seen += [(2 * cb + h, b, 2 * t + j) for h in (0, 1) for j in (0, 1) if 2 * t + j < n64]
+        elif k.startswith("nsrk_conv1d_ps"):
+            mt = int(k[len("nsrk_conv1d_ps")])
+            cols = n64 * B - n
+            assert (gy, gz, block) == (1, 1, 256) and gx == cols * -(-C_out // (64 * mt))
+            for tile in range(gx):
+                cb, ct = divmod(tile, cols)
+                b, t = divmod(n + ct, n64)
+                seen += [(mt * cb + m, b, t) for m in range(mt)]
+    return seen
+
+
+def test_record_launches_cover_the_output_once(routes):
+    cases = []
+    for C_out in (2, 64, 96, 128, 130, 200, 256, 384):
+        for B in (1, 2, 3, 8):
+            for T in (1, 63, 65, 128, 129, 400, 1001, 4096, 8224, 16384, 16449, 21920, 33000, 57601):
+                for K, dil in ((7, 1), (11, 5)):
+                    cases.append((("stats", 128, C_out, B, T, K, dil, True), B, T, C_out))
+    for (c, B, T, C_out), (st, log) in zip(cases, routes([_conv(*c[0]) for c in cases])):
+        assert st == 0, c
+        if _family(log) != "records":
+            continue
+        blocks = range(2 * -(-C_out // 128))
+        want = {(cb, b, t) for cb in blocks for b in range(B) for t in range(-(-T // 64))}
+        seen = _record_columns(log, B, T, C_out)
+        live = {(cb, b, t) for cb, b, t in want if 64 * cb < C_out}
+        assert len(seen) == len(set(seen)), c
+        assert live <= set(seen) <= want, c
