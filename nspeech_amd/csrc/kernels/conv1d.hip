@@ -1918,9 +1918,11 @@ NSR_DEV void sum2_256(double& a, double& b, double* red) {
  * result does not depend on timing.
  * What the f32 blocks cannot give is taken from the row itself, read once more: a sum of squares that overflowed
  * in a block, a variance too small for f32 squares (with eps as small), and, for rows whose statistics a pass
- * over the output used to take (`reread`: rows that are not whole 16-byte vectors), mean^2 > 4 var, where the
- * rounding of the block means shows: at |mean| = 1000 std 1 / sqrt(var) was off by 2e-6 at T = 2401, against
- * 1e-7. */
+ * over the output used to take (`reread`: rows that are not whole 16-byte vectors), mean^2 > nblk var / 2. The
+ * rounding of the block means (u |mean| each) moves var by about 0.35 u |mean| std / sqrt(nblk) then, under half of
+ * what rounding var to f32 does; at |mean| = 1000 std 1 / sqrt(var) was off by 2e-6 at T = 2401, against 1e-7.
+ * (With 4 var in place of nblk var / 2, [1, 128, 57601] K = 3 with biases of the output's spread took 45.8 us
+ * against 36.4: one row in twenty was read again, by one workgroup each.) */
 extern "C" __global__ void __launch_bounds__(256) nsrk_conv_rowstats_merge(const nsr_rowstats_args a) {
   __shared__ double red[2][8];
   const int tid = threadIdx.x;
@@ -1944,7 +1946,7 @@ extern "C" __global__ void __launch_bounds__(256) nsrk_conv_rowstats_merge(const
   }
   sum2_256(s1, s2, red[0]);
   double mean = p + s1 / T, var = (s2 - s1 * s1 / T) / T;
-  if (!(var < 1e300) || (float)var + a.eps < 1e-30f || (a.reread && mean * mean > 4.0 * var)) { /* workgroup-uniform */
+  if (!(var < 1e300) || (float)var + a.eps < 1e-30f || (a.reread && mean * mean > 0.5 * a.nblk * var)) { /* workgroup-uniform */
     const float* x = a.x + row * a.T_out;
     p = fabs(mean) < 1e300 ? mean : 0.0;
     s1 = 0.0;

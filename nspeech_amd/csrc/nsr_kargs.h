@@ -188,7 +188,7 @@ typedef struct nsr_rowstats_args {
   int32_t nblk;
   int32_t T_out;           /* block i holds min(32, T_out - 32 i) columns */
   float eps;
-  int32_t reread;          /* 1: rows with mean^2 > 4 var are read again (see nsrk_conv_rowstats_merge) */
+  int32_t reread;          /* 1: rows of a large mean are read again (see nsrk_conv_rowstats_merge) */
 } nsr_rowstats_args;
 
 typedef struct nsr_conv_pack_args {
