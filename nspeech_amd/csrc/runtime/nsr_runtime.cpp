@@ -1511,6 +1511,8 @@ ConvSize conv_size(const nsr_conv_args& a, bool fused) {
 //   fused: 128 -> 128 K = 3, 256 tiles 17.6 / 19.5; 64 -> 64 K = 5, 512 tiles 26.4 / 24.5
 //   plain: 128 -> 128 K = 3, 16 tiles 16.1 / 15.3; K = 5, 64 tiles 19.3 / 22.6, 512 tiles 28.4 / 26.2;
 //     64 -> 64 K = 5, 1024 tiles 31.4 / 38.8; 512 -> 32 K = 5, 64 tiles 39.0 / 34.6, 512 tiles 56.3 / 65.3
+// With a residual, which the fallback kernel's epilogue reads element by element: 128 -> 128 K = 3, 16 / 256 tiles fused
+// 19.2 / 19.1, 21.0 / 20.2; 64 -> 64 K = 3, 512 tiles plain 16.1 / 14.4; K = 7, 512 tiles fused 33.6 / 28.3.
 // Over all of them the choice costs 0.3% on average against the better one, at most 27% (narrow channels, 5 to 9 us).
 // Where only the input's rows are ragged (an even K, padding on one side) the fallback kernel stores 16-byte vectors and
 // is about 14% faster than that: 128 -> 128 K = 2, 64 tiles plain 12.8 / 14.5, fused 12.3 / 17.7; K = 4, 1024 tiles plain
@@ -1523,12 +1525,16 @@ bool conv_fallback_faster(const nsr_conv_args& a, bool fused, int64_t n_cu) {
     return !(s.tiles > (s.two ? 3 : 1) * n_cu && a.C_in >= 64 && (a.K <= 3 || (s.two ? s.full : s.wide)));
   }
   if (s.n_ch > 1) return s.two && s.tiles > n_cu && (a.C_out <= 64 || s.n_ch >= 4);
+  const bool res = a.residual != nullptr;
   if (s.tiles > n_cu) {
-    if (a.K <= 3 && !s.two) return false;
+    if ((a.K <= 3 && !s.two) || (res && a.C_in >= 64 && (a.K <= 3 || !s.two))) return false;
     return !(s.two && a.K > 3 ? s.full : s.wide || (a.C_in >= 64 && s.tiles > 3 * n_cu));
   }
   if (a.K > 3) return true;
-  if (fused) return !(a.row_part && (s.full ? 4 * s.tiles >= n_cu : s.wide && a.C_out > 64 && 2 * s.tiles >= n_cu));
+  if (fused && res && a.C_in >= 64 && a.C_out > 96 && (a.K <= 2 || (s.full && s.n_co == 1))) return false;
+  if (fused)  // the statistics pass takes a workgroup per row, however short
+    return !(a.row_part && (s.full ? 4 * s.tiles >= n_cu || (int64_t)a.B * a.C_out >= 2 * n_cu
+                                   : s.wide && a.C_out > 64 && 2 * s.tiles >= n_cu));
   return !(s.n_co == 1 && a.C_out > 96 && a.C_in >= 64);
 }
 

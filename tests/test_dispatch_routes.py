@@ -154,6 +154,7 @@ def _family(log):
     ("plain", 128, 128, 1, 2401, 7, 1, True, "records"), ("stats", 128, 128, 1, 19201, 7, 5, True, "records"),
     ("stats", 128, 128, 4, 57601, 11, 5, True, "records"), ("plain", 64, 64, 4, 8189, 7, 1, True, "fallback"),
     ("plain", 32, 32, 4, 8189, 7, 1, True, "fallback"), ("plain", 64, 64, 4, 1021, 7, 1, True, "records"),
+    ("stats", 128, 128, 8, 401, 3, 5, True, "one launch"),
     # ragged inputs of an even K, outputs of whole vectors
     ("plain", 128, 128, 4, 1025, 2, 1, True, "fallback"), ("fused", 256, 256, 1, 1021, 2, 1, True, "fallback"),
     ("fused", 128, 128, 4, 16381, 2, 1, True, "one launch"), ("plain", 256, 256, 4, 4097, 2, 1, True, "fallback"),
@@ -162,6 +163,14 @@ def _family(log):
     ("stats", 128, 128, 8, 115200, 3, 5, True, "one launch"), ("stats", 256, 256, 1, 3200, 11, 3, True, "records")])
 def test_conv_takes_the_faster_kernels(routes, mode, C_in, C_out, B, T, K, dil, records, family):
     (st, log), = routes([_conv(mode, C_in, C_out, B, T, K, dil, records)])
+    assert st == 0 and _family(log) == family, log
+
+
+@pytest.mark.parametrize("mode,C_in,C_out,B,T,K,dil,family", [
+    ("fused", 128, 128, 4, 4093, 3, 1, "one launch"), ("stats", 128, 128, 1, 401, 3, 1, "one launch"),
+    ("fused", 64, 64, 4, 8189, 7, 1, "one launch"), ("fused", 128, 128, 4, 1021, 5, 1, "fallback")])
+def test_ragged_conv_with_a_residual(routes, mode, C_in, C_out, B, T, K, dil, family):
+    (st, log), = routes([_conv(mode, C_in, C_out, B, T, K, dil, False, res=True)])
     assert st == 0 and _family(log) == family, log
 
 
