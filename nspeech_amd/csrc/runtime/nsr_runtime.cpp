@@ -1538,14 +1538,48 @@ bool conv_fallback_faster(const nsr_conv_args& a, bool fused, int64_t n_cu) {
   return !(s.n_co == 1 && a.C_out > 96 && a.C_in >= 64);
 }
 
-// Such rows with K >= 7 (rows of whole vectors: always): is the record path faster than both? Its records hold whole
-// 128-channel blocks, written and read whatever C_in is. Fallback / records, as above: 128 -> 128 K = 7, 64 tiles fused
-// 21.3 / 15.1, plain 22.0 / 16.0, 1024 tiles fused 86.2 / 54.6, plain 59.3 / 56.3; 64 -> 64 K = 7, 64 tiles plain
-// 16.8 / 15.2, 512 tiles 20.8 / 28.2 (fused 30.2 / 28.0); 32 -> 32 K = 7, 64 tiles fused 13.3 / 14.5, plain 14.2 / 15.0.
-bool conv_records_faster_ragged(const nsr_conv_args& a, bool fused, int64_t n_cu) {
+// Is the record path faster than both? MI355X, us per graph replay.
+// K >= 7: always with output rows of whole vectors. With others (fallback / records): its records hold whole
+// 128-channel blocks, written and read whatever C_in is: 128 -> 128 K = 7, 64 tiles fused 21.3 / 15.1, plain 22.0 / 16.0,
+// 1024 tiles fused 86.2 / 54.6, plain 59.3 / 56.3; 64 -> 64 K = 7, 64 tiles plain 16.8 / 15.2, 512 tiles 20.8 / 28.2 (fused
+// 30.2 / 28.0); 32 -> 32 K = 7, 64 tiles fused 13.3 / 14.5, plain 14.2 / 15.0.
+// K = 3 to 6 with several 128-channel blocks (one-launch / records): the records pass and its launch, and writing and
+// reading the records, against one-launch tiles that leave CUs idle, transform the input once per output block (only
+// several output blocks do that, and only fused inputs cost much there) and hold one block's weights at a time.
+//   128 -> 256 K = 3, 64 / 256 / 512 tiles fused 20.9 / 11.9, 22.4 / 17.5, 22.9 / 23.7, 2048 tiles 63.8 / 56.9, with
+//     statistics 70.8 / 75.1; plain 18.5 / 12.6, 20.4 / 18.1, 21.6 / 24.4, 56.8 / 58.1
+//   256 -> 128 K = 3, 64 / 128 / 320 / 512 / 2048 tiles fused 21.0 / 16.6, 21.3 / 21.8, 37.1 / 28.9, 39.5 / 38.7,
+//     124 / 129; plain 18.2 / 17.5, 18.4 / 22.6, 30.9 / 32.6, 33.8 / 39.7, 99.2 / 130
+//   256 -> 256 K = 3, 96 / 256 / 512 / 2048 tiles fused 20.7 / 16.4, 23.1 / 24.3, 38.0 / 31.1, 118 / 100; plain 18.6 / 17.4,
+//     20.9 / 25.4, 32.7 / 33.8, 98.1 / 104; K = 5 plain, 512 / 2048 tiles 41.9 / 40.0, 134 / 121
+//   512 -> 512 K = 3, 800 tiles plain 93.2 / 75.4
+//   a last round part full: 128 -> 256 K = 5, 1600 tiles with statistics 84.2 / 69.9 (2048 tiles 87.5 / 87.9); 256 -> 128
+//     K = 5, 2400 tiles fused 195 / 168 (2048 tiles 157 / 150)
+// One 128-channel block each way: one-launch (two dilations of a ResBlock at K = 3, [4, 128, 57600] 468 us against
+// 595 us on records, [1, 128, 19200] 110 us on both).
+bool conv_records_faster(const nsr_conv_args& a, bool fused, int64_t n_cu) {
   const ConvSize s = conv_size(a, fused);
-  if (s.two) return s.full || (s.wide && s.tiles <= n_cu) || (a.C_in >= 64 && 2 * s.tiles <= n_cu);
-  return s.wide || (a.C_in >= 64 && (2 * s.tiles <= n_cu || s.tiles > 3 * n_cu)) || 16 * s.tiles <= n_cu;
+  if (a.K >= 7) {
+    if (conv_out16(a)) return true;
+    if (s.two) return s.full || (s.wide && s.tiles <= n_cu) || (a.C_in >= 64 && 2 * s.tiles <= n_cu);
+    if (s.wide || 16 * s.tiles <= n_cu) return true;
+    return a.residual ? a.C_in >= 64 || s.tiles > 3 * n_cu : a.C_in >= 64 && (2 * s.tiles <= n_cu || s.tiles > 3 * n_cu);
+  }
+  if (a.K < 3 || (s.n_ch == 1 && s.n_co == 1)) return false;
+  // the one-launch kernels' last round is as long as a full one: how much of its rounds a shape fills, in 32nds
+  const int64_t rounds = (s.tiles + n_cu - 1) / n_cu;
+  auto fills = [&](int n) { return 32 * s.tiles > n * n_cu * rounds; };
+  if (s.n_ch == 1) {
+    // narrow inputs and ragged rows into whole vectors: the fallback kernel is the faster one from half a round on
+    const bool half = !conv_rows16(a) && !a.residual && (a.C_in < 64 || conv_out16(a));
+    if (s.tiles <= 2 * n_cu) return s.tiles <= (half ? n_cu / 2 : n_cu);
+    return a.K >= 5 || (fused && (!a.row_part || !fills(31))) || !fills(28);
+  }
+  const int64_t few = fused ? s.n_ch + (s.n_co > 1 ? 3 : 1) : s.n_ch + (s.n_co > 1 ? 1 : 0);  // eighths of a round
+  if (8 * s.tiles <= few * n_cu) return true;
+  if (s.tiles <= n_cu) return false;
+  if (s.n_co > 1) return fused || s.n_co >= 4 || a.K >= 5;
+  return fused && (a.K >= 5 ? s.tiles > 3 * n_cu || !fills(30) : !fills(a.row_part ? 28 : 30));
 }
 
 nsr_status conv_launch(bool fused, nsr_conv_args& a, nsr_stream_t stream, const char* what, bool* emitted = nullptr) {
@@ -1638,14 +1672,8 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   const int64_t D = (int64_t)(a.K - 1) * a.dilation;
   const int64_t TLe = kCvTW + D + (D & 1);
   // TLe <= 184 leaves 72 ring slots outside a window, which with the 56 rows after the ring stage a 128-row tile.
-  // Below K = 7 with one 128-channel block each way the records pass (x read, records written) costs more than
-  // the one-launch kernels lose to their per-element work (measured on MI355X, two dilations of a ResBlock at
-  // K = 3: [4, 128, 57600] 468 us against 595 us on records, [1, 128, 19200] 110 us on both). With more blocks the
-  // one-launch kernel transforms its input once per output block and the records win from K = 3:
-  // [8, 256, 9600] 571 against 639 us, [4, 256, 3200] 147 against 173 us, [1, 256, 3200] 87 against 110 us.
-  const bool blocks1 = a.C_in <= kCvCI && a.C_out <= kCvCO;
-  if (!records || a.K < (blocks1 ? 7 : 3) || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0 ||
-      (a.K >= 7 && !conv_out16(a) && !conv_records_faster_ragged(a, fused, dm->n_cu)))
+  if (!records || TLe > 184 || a.C_out % 2 != 0 || kCvRingLds > dm->max_lds || a.T_in <= 0 ||
+      !conv_records_faster(a, fused, dm->n_cu))
     return conv_launch(fused, a, stream, what, emitted);
   const int64_t Tp = (int64_t)a.T_in + 2 * a.padding;
   const int64_t n_ch = (a.C_in + 127) / 128, n_co = (a.C_out + 127) / 128;

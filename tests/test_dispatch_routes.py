@@ -158,6 +158,16 @@ def _family(log):
     # ragged inputs of an even K, outputs of whole vectors
     ("plain", 128, 128, 4, 1025, 2, 1, True, "fallback"), ("fused", 256, 256, 1, 1021, 2, 1, True, "fallback"),
     ("fused", 128, 128, 4, 16381, 2, 1, True, "one launch"), ("plain", 256, 256, 4, 4097, 2, 1, True, "fallback"),
+    # K = 3 to 6 with several channel blocks: records where they win
+    ("stats", 256, 256, 1, 3200, 3, 1, True, "records"), ("stats", 256, 256, 8, 9600, 3, 5, True, "records"),
+    ("fused", 256, 256, 4, 2048, 3, 1, True, "one launch"), ("plain", 256, 256, 4, 2048, 3, 1, True, "one launch"),
+    ("plain", 256, 128, 8, 9600, 3, 1, True, "one launch"), ("stats", 256, 128, 8, 9600, 3, 1, True, "one launch"),
+    ("plain", 512, 32, 4, 3200, 3, 1, True, "one launch"), ("fused", 256, 128, 4, 5120, 3, 1, True, "records"),
+    ("plain", 128, 256, 4, 4096, 3, 1, True, "one launch"), ("plain", 128, 256, 4, 512, 3, 1, True, "records"),
+    ("stats", 128, 256, 8, 6400, 5, 1, True, "records"), ("stats", 128, 256, 4, 12288, 3, 1, True, "one launch"),
+    ("stats", 128, 256, 4, 9600, 3, 1, True, "records"),
+    ("fused", 256, 128, 8, 19200, 5, 1, True, "records"), ("fused", 256, 128, 4, 12288, 5, 1, True, "one launch"),
+    ("plain", 512, 512, 4, 3200, 3, 1, True, "records"), ("plain", 256, 256, 4, 16384, 5, 1, True, "records"),
     # rows of whole vectors keep the kernels they had
     ("plain", 16, 16, 4, 400, 3, 1, True, "one launch"), ("plain", 32, 32, 4, 8188, 7, 1, True, "records"),
     ("stats", 128, 128, 8, 115200, 3, 5, True, "one launch"), ("stats", 256, 256, 1, 3200, 11, 3, True, "records")])
