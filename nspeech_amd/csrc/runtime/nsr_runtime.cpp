@@ -1700,7 +1700,14 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
   // 14 tiles 184 / 115 / 125, 50 282 / 181 / 196, 76 138 / 111 / 102, 100 161 / 132 / 126, 151 193 / 191 / 195,
   // 200 187 / 206 / 191, 226 149 / 151 / 145, 280 386 / 322 / 338, 302 241 / 211 / 219, 452 286 / 300 / 298.
   // MT = 1 (four times the tiles) while they fit one per CU, and past one round of the large tiles.
+  // With two channel chunks the line in one round is where MT = 2 (twice the tiles) fits one per CU: 160 tiles K = 7, 256
+  // channels 40.4 us a stage against 43.8 for MT = 2 (130 tiles 40.1 / 41.9), while 128 channels take 33.7 against 32.9 and
+  // 512 channels 67.9 against 66.9. In the second of two rounds one chunk stops earlier, where a longer window leaves
+  // fewer small workgroups on a CU: K = 11 dilation 5, 340 tiles, 128 channels 58.6 against 60.5, 256 channels 95.8
+  // against 93.4.
   const int64_t rounds = (tiles + dm->n_cu - 1) / dm->n_cu;
+  const int64_t small_limit = rounds == 1 ? (n_ch == 2 ? dm->n_cu / 2 : dm->n_cu * 7 / 10)
+                                          : (n_ch == 1 ? 2 * dm->n_cu * 5 / 8 : 2 * dm->n_cu * 7 / 10);
   static const KId ps[2][2][2] = {{{K_nsrk_conv1d_ps1_f16x2, K_nsrk_conv1d_ps1_f16x2_st},
                                    {K_nsrk_conv1d_ps1_res_f16x2, K_nsrk_conv1d_ps1_res_f16x2_st}},
                                   {{K_nsrk_conv1d_ps2_f16x2, K_nsrk_conv1d_ps2_f16x2_st},
@@ -1712,15 +1719,17 @@ static nsr_status conv_records(bool fused, nsr_conv_args& a, char* records, nsr_
     void* pq[] = {&a, &xs, &wf, &ct0};
     return launch(ps[mt - 1][a.residual != nullptr][stats], (unsigned)grid, 1, 256, slots * 1040, stream, pq);
   };
-  if (rounds <= 2 && 10 * tiles <= 7 * rounds * dm->n_cu)
+  if (rounds <= 2 && tiles <= small_limit)
     return small_tiles(4 * tiles <= dm->n_cu || rounds == 2 ? 1 : 2, 0);
-  // A last round that fills at most a third of the chip goes to the small-tile kernel in a launch of its own
-  // (whole columns of channel blocks). Measured, us per ResBlock, one launch / two: [8, 256, 4200] K = 11 (528
+  // A last round that fills at most a third of the chip (a quarter with one channel chunk: [4, 128, 18560] K = 7, 580 tiles,
+  // 73.3 us a stage in one launch, 75.4 in two; 560 tiles 72.8 and 71.8) goes to the small-tile kernel in a launch of its
+  // own (whole columns of channel blocks). Measured, us per ResBlock, one launch / two: [8, 256, 4200] K = 11 (528
   // tiles) 568 / 534, [5, 128, 26400] K = 7 (1035) 474 / 467, [4, 128, 57601] K = 11 (1804) 1405 / 1390.
   int n_tiles = (int)tiles;
   const int64_t rest = tiles % dm->n_cu;
   // (the small-tile kernel's 32-bit offsets of whole channel blocks must not wrap)
-  if (rounds > 2 && rest > 0 && 3 * rest <= dm->n_cu && 4 * n_co * kCvCO * ((int64_t)a.T_out + kCvTW) <= kConvMaxSlabBytes)
+  if (rounds > 2 && rest > 0 && (n_ch == 1 ? 4 : 3) * rest <= dm->n_cu &&
+      4 * n_co * kCvCO * ((int64_t)a.T_out + kCvTW) <= kConvMaxSlabBytes)
     n_tiles = (int)((tiles - rest) / n_co * n_co);
   // one workgroup per CU, a multiple of 8 (the kernel's XCD split), never fewer than there are tiles below that:
   // rounded down, 151 tiles gave some of 144 workgroups a second tile (256 against 193 us per ResBlock)

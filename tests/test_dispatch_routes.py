@@ -184,6 +184,19 @@ def test_ragged_conv_with_a_residual(routes, mode, C_in, C_out, B, T, K, dil, fa
     assert st == 0 and _family(log) == family, log
 
 
+@pytest.mark.parametrize("C,B,T,K,dil,kernels", [
+    (128, 1, 128 * 64, 7, 1, ["ps1"]), (128, 1, 128 * 65, 7, 1, ["ps2"]), (128, 1, 128 * 179, 7, 1, ["ps2"]),
+    (128, 1, 128 * 180, 7, 1, ["pr"]), (256, 1, 128 * 64, 7, 1, ["ps2"]), (256, 1, 128 * 65, 7, 1, ["pr"]),
+    (256, 4, 2400, 11, 1, ["pr"]), (512, 1, 128 * 40, 7, 1, ["ps2"]), (128, 1, 128 * 320, 11, 5, ["ps1"]),
+    (128, 1, 128 * 321, 11, 5, ["pr"]), (256, 1, 128 * 179, 7, 1, ["ps1"]), (128, 1, 128 * 576, 7, 1, ["pr", "ps1"]),
+    (128, 1, 128 * 577, 7, 1, ["pr"]), (256, 1, 128 * 298, 7, 1, ["pr", "ps1"]), (256, 1, 128 * 299, 7, 1, ["pr"])])
+def test_record_tiles(routes, C, B, T, K, dil, kernels):
+    """64 x 64, 128 x 64 (ps1, ps2) or 128 x 128 tiles (pr), or the last, a third at most filled round on small ones."""
+    (st, log), = routes([_conv("stats", C, C, B, T, K, dil, True)])
+    assert st == 0
+    assert [l[0].split("_")[2] for l in log if l[0].startswith("nsrk_conv1d_p")] == kernels, log
+
+
 def _record_columns(log, B, T_out, C_out):
     """The 64-column tiles of the output that a record call's launches write, as (channel block of 64, batch, tile)."""
     n64, n128, seen = -(-T_out // 64), -(-T_out // 128), []
