@@ -416,7 +416,7 @@ def _conv_tout(T, K, padding, dilation):
 WS_PACKED_WEIGHTS, WS_IN_STATS, WS_OUT_STATS, WS_RECORDS = 1, 2, 4, 8
 
 
-@functools.lru_cache(maxsize=1024)
+@functools.lru_cache(maxsize=1024, typed=True)  # typed: 3.0 must not find the entry of 3, it is no argument of the call
 def conv1d_workspace_bytes(B, C_in, C_out, T, K, padding, dilation, parts) -> int:
     """Bytes of device workspace a conv entry point of this shape needs for `parts` (WS_* flags ORed)."""
     n = C.c_int64(0)

@@ -202,3 +202,12 @@ def test_conv_rows_past_a_buffer_descriptor_are_unsupported():
     assert "buffer descriptor" in L.nsr_last_error().decode()
     assert packed(0, 16, 1024, 1 << 20) == abi.NSR_ERR_UNSUPPORTED     # output rows: 4 * 1024 * 2^20 = 2^32
     assert packed(0, 16, 1023, 1 << 20) == abi.NSR_OK
+
+
+def test_workspace_bytes_refuses_a_float_also_after_the_integer_call():
+    """The sizes are remembered by argument, and 400.0 == 400 with the same hash."""
+    args = (1, 128, 128, 400, 7, 3, 1, abi.WS_RECORDS)
+    n = abi.conv1d_workspace_bytes(*args)
+    assert n > 0 and abi.conv1d_workspace_bytes(*args) == n
+    with pytest.raises((C.ArgumentError, TypeError)):
+        abi.conv1d_workspace_bytes(*(float(v) if v == 400 else v for v in args))
