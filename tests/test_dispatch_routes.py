@@ -9,6 +9,9 @@ from pathlib import Path
 
 import pytest
 
+from .test_gpu_adain_ragged_rows import ROW_SLOTS, slot_lengths
+from .test_gpu_conv_record_tiles import SHAPES as RECORD_TILE_SHAPES
+
 ROOT = Path(__file__).resolve().parent.parent
 LIB = ROOT / "nspeech_amd" / "lib" / "libnspeech_rocm.so"
 CUS, LDS = 256, 163840
@@ -194,7 +197,20 @@ def test_record_tiles(routes, C, B, T, K, dil, kernels):
     """64 x 64, 128 x 64 (ps1, ps2) or 128 x 128 tiles (pr), or the last, a third at most filled round on small ones."""
     (st, log), = routes([_conv("stats", C, C, B, T, K, dil, True)])
     assert st == 0
-    assert [l[0].split("_")[2] for l in log if l[0].startswith("nsrk_conv1d_p")] == kernels, log
+    assert _tiles(log).split("+") == kernels, log
+
+
+def _tiles(log):
+    return "+".join(l[0].split("_")[2] for l in log if l[0].startswith("nsrk_conv1d_p") and l[0] != "nsrk_conv1d_pack")
+
+
+def test_record_tile_shapes_take_the_kernels_they_name(routes):
+    for mode in ("stats", "fused"):
+        calls = [_conv(mode, ci, co, B, T, K, dil, True, res) for B, ci, co, T, K, dil, res, _ in RECORD_TILE_SHAPES]
+        one = [_conv(mode, ci, co, B, T, K, dil, False, res) for B, ci, co, T, K, dil, res, _ in RECORD_TILE_SHAPES]
+        for shape, (st, log), (st1, log1) in zip(RECORD_TILE_SHAPES, routes(calls), routes(one)):
+            assert st == 0 and _tiles(log) == shape[-1], (shape, log)
+            assert st1 == 0 and _family(log1) == "one launch", (shape, log1)  # both emit the statistics
 
 
 def _record_columns(log, B, T_out, C_out):
@@ -236,3 +252,49 @@ def test_record_launches_cover_the_output_once(routes):
         live = {(cb, b, t) for cb, b, t in want if 64 * cb < C_out}
         assert len(seen) == len(set(seen)), c
         assert live <= set(seen) <= want, c
+
+
+def _listed(pattern):
+    text = (ROOT / "nspeech_amd" / "csrc" / "runtime" / "nsr_kernels.def").read_text()
+    return {k for k in re.findall(r"NSR_KERNEL\(\w+, (\w+)\)", text) if re.match(pattern, k)}
+
+
+def test_every_ragged_row_kernel_is_run_by_a_test(routes):
+    lengths = [T for s in ROW_SLOTS for T in slot_lengths(s)]
+    seen = {log[0][0] for _, log in routes([_adain(3, T) for T in lengths])}
+    assert _listed(r"nsrk_adain_rowu_") <= seen, sorted(_listed(r"nsrk_adain_rowu_") - seen)
+
+
+def test_every_listed_adain_and_conv_kernel_is_reached(routes):
+    """No kernel that nothing launches: rows of every slot count on both sides of 16-byte alignment, and convs over the
+    shapes that the rules tell apart."""
+    calls = [_adain(r, T, off) for r in (3, 300) for T in _lengths() for off in (0, 4)]
+    for mode in ("stats", "fused", "plain"):
+        for res in (False, True):
+            for records in (False, True):
+                for ci, co in ((16, 16), (128, 128), (256, 256)):
+                    for K, dil in ((1, 1), (3, 1), (3, 5), (2, 40), (3, 32), (5, 1), (7, 5), (11, 5)):
+                        for B, T in ((1, 401), (1, 3200), (1, 19200), (1, 19201), (4, 57600), (4, 57601)):
+                            for pad in {(K - 1) * dil // 2, (K - 1) * dil // 2 + 1}:
+                                calls.append(_conv(mode, ci, co, B, T, K, dil, records, res, pad=pad))
+    # plain with a residual or statistics: nsr_conv1d_f16w_packed and its form with statistics
+    for K, dil in ((1, 1), (3, 1), (2, 40), (7, 5), (11, 5)):
+        for stats in (False, True):
+            for res in (False, True):
+                for T in (3200, 57600):
+                    calls.append(_packed(128, 4, T, K, dil, stats, res))
+    seen = {l[0] for st, log in routes(calls) for l in log}
+    want = _listed(r"nsrk_(adain_row_b|adain_rowu|adain_res|adain_long|adain_stats|conv)")
+    assert want <= seen, sorted(want - seen)
+
+
+def _packed(C, B, T, K, dil, stats, res):
+    pad = (K - 1) * dil // 2
+    T_out = T + 2 * pad - dil * (K - 1)
+    a = [("p", 1 << 40), ("p", 256), ("p", 0), ("p", 3 << 40 if res else 0), ("p", 2 << 40)]
+    sh = [("l", B), ("l", C), ("l", C), ("l", T), ("l", K), ("l", pad), ("l", dil)]
+    if not stats:
+        return ["nsr_conv1d_f16w_packed", [*a, *sh, ("p", 0)]]
+    need = -(-8 * B * C * -(-T_out // 32) // 256) * 256
+    return ["nsr_conv1d_f16w_packed_stats", [*a, ("p", 256), *sh, ("f", 1e-5), ("p", 1 << 47),
+                                             ("l", need), ("p", 0)]]

@@ -111,7 +111,8 @@ def _bucket_lengths():
     aligned rows (T % 4 == 0) in 16-byte chunks: 256 threads x 1..8 slots,
     512 threads x {5..20} VGPR slots (rows of up to 19 slots), 512 x (1..39
     VGPR + 19 LDS slots) for rows of 20..58 slots, one kernel per slot count,
-    then the long-row kernel; unaligned rows (T % 4 != 0) by interior-chunk count."""
+    then the long-row kernel; rows of T % 4 != 0 by interior-chunk count, on the row kernel's ragged form or the kernel of
+    one workgroup per row (every variant of both: test_gpu_adain_ragged_rows.py)."""
     Ts = set()
     for nv in range(1, 9):                                       # b256 row kernels
         Ts |= {4 * 256 * nv, 4 * (256 * (nv - 1) + 1)}
@@ -123,7 +124,7 @@ def _bucket_lengths():
     for ns in range(20, 59):                                      # b512, 19 LDS slots + ns - 19 VGPR slots
         Ts |= {4 * 512 * ns, 4 * (512 * (ns - 1) + 1)}
     Ts |= {4 * (512 * 58 + 1), 150000}                            # long-row kernel
-    for need in (1, 256, 257, 1536, 1537, 2048, 2049, 6144, 8192, 8193, 12288, 16384, 16385):  # unaligned
+    for need in (1, 256, 257, 1536, 1537, 2048, 2049, 6144, 8192, 8193, 12288, 16384, 16385):  # T % 4 != 0
         Ts.add(4 * need + 5)
     return sorted(Ts)
 

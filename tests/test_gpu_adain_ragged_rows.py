@@ -61,6 +61,46 @@ def test_f16_rows(B, C, T):
     _run(B, C, T, torch.float16, RTOL_F16, B + C + T)
 
 
+# A length in every slot count of the row kernel's ragged form that its rule takes with few rows: 512 chunks of 16 bytes
+# a slot, both ends of the slot count of one kernel (test_dispatch_routes.py checks that every such kernel is among them).
+ROW_SLOTS = [5, 6, 7, 8, 9, 10] + list(range(13, 59))
+
+
+def slot_lengths(slots):
+    """The longest row of `slots` slots and the shortest of slots - 1 .. slots, neither a multiple of 4."""
+    return 4 * (512 * slots + 2) - 3, 4 * (512 * (slots - 1) + 3) + 1
+
+
+@pytest.mark.parametrize("slots", ROW_SLOTS)
+def test_f32_every_slot_count(slots):
+    for T in slot_lengths(slots):
+        say("adain ragged f32 slots", slots, T)
+        _run(1, 3, T, torch.float32, RTOL_F32, T)
+
+
+@pytest.mark.parametrize("T", [500, 8197, 12000, 24000, 24001, 32771, 48001, 49152, 65000, 65536, 70001, 118784, 131073])
+@pytest.mark.parametrize("shift_x,shift_out", [(1, 1), (1, 0), (0, 3)])
+def test_f32_misaligned_views(T, shift_x, shift_out):
+    """x or out 4 to 12 bytes past a 16-byte boundary: the one-row-per-workgroup kernels over their whole range of
+    lengths, and the two-read kernel past it."""
+    say("adain misaligned f32", T, shift_x, shift_out)
+    g = configs.rng(T + 16 * shift_x + shift_out)
+    B, C = 2, 3
+    n = B * C * T
+    xb = torch.from_numpy(g.standard_normal(n + 8, dtype=np.float32)).cuda()
+    x = xb[shift_x:shift_x + n].view(B, C, T)
+    x[:, 1] += 3.0  # the centred pass
+    buf = torch.full((n + 32,), -7.0, device="cuda")
+    out = buf[16 + shift_out:16 + shift_out + n].view(B, C, T)
+    gam, bet = (torch.from_numpy((g.standard_normal((B, C)) * 0.1).astype(np.float32)).cuda() for _ in range(2))
+    alp = torch.from_numpy(g.uniform(0.5, 1.5, C).astype(np.float32)).cuda()
+    abi.adain_snake(x, gam, bet, alp, out=out)
+    lo, hi = 16 + shift_out, 16 + shift_out + n
+    assert bool((buf[:lo] == -7.0).all()) and bool((buf[hi:] == -7.0).all()), "wrote outside the output"
+    ref = _closed_form(x, gam, bet, alp)
+    assert float(((out.double() - ref).abs() / ref.abs().clamp_min(1.0)).max()) <= RTOL_F32
+
+
 @pytest.mark.parametrize("T", [65543, 70001, 90002, 115201, 118790, 118797])
 def test_f32_statistics_range(T):
     """Rows past the reach of the one-row-per-workgroup kernel keep statistics in f64: no overflow of the squares

@@ -49,12 +49,12 @@ def _reference(x, gam, bet, alp, w, bias, res, pad, dil):
     (2, 256, 256, 255, 7, 1, False),    # two channel chunks and blocks
     (1, 144, 200, 601, 9, 5, True),     # partial channel chunk and block
     (3, 64, 96, 1001, 8, 1, True),      # odd (K - 1) dilation
-    (1, 128, 128, 19201, 11, 5, True),  # many tiles per workgroup are not reached; tiles past one per CU are below
+    (1, 128, 128, 19201, 11, 5, True),
     (2, 128, 128, 19203, 7, 5, True),
     (3, 128, 128, 128 * 257 - 63, 7, 1, True),   # three rounds of tiles and a rest of 3, a half tile at each row's end
     (2, 256, 256, 128 * 130 + 5, 7, 3, True),    # two channel blocks, a rest of 12 across the last batch
     (3, 128, 128, 128 * 171 + 32, 7, 1, False),  # a rest that starts inside the last batch, whole 32-column blocks
-    (1, 64, 64, 601, 5, 2, True),       # K < 7: the one-launch kernels
+    (1, 64, 64, 601, 5, 2, True),       # K < 7: mostly without records
     (2, 128, 128, 1003, 3, 5, True),
     (1, 128, 128, 19201, 3, 1, False),
     (1, 256, 128, 333, 5, 3, True),
@@ -125,7 +125,8 @@ def test_ragged_rows_from_misaligned_views():
 
 @pytest.mark.parametrize("C,T,K,dil,pad,res", [
     (128, 1, 1, 1, 0, False), (16, 63, 1, 1, 5, True), (128, 200, 2, 1, 1, True), (96, 517, 3, 1, 1, True),
-    (128, 64, 3, 32, 32, True),   # the widest halo: 64 columns shared between tiles
+    (128, 64, 3, 32, 32, True),   # 64 columns shared between tiles (past this kernel's LDS: the streamed-weight kernel)
+    (128, 3000, 3, 20, 19, False), (128, 3001, 2, 40, 21, False), (128, 130, 3, 18, 17, True),  # windows past 96 columns
     (128, 131, 3, 5, 70, True),   # padding wider than a tile
     (64, 1000, 2, 7, 0, False), (128, 40000, 3, 3, 3, True),
 ])
@@ -182,3 +183,82 @@ def test_row_statistics_of_ragged_rows(C_out, T, K):
             em = ((st[:, 0] - m).abs() / (2.0 ** -24 * m.abs() + 2.0 ** -22 * sd)).max()
             er = (st[:, 1] * sd - 1.0).abs().max() / (10 * 2.0 ** -24)
             assert em <= 1.0 and er <= 1.0, f"std {std} mean {mean} records={records}: {em:.2f}, {er:.2f} of the bars"
+
+
+@pytest.mark.parametrize("C_in,C_out,T,K,dil,pad", [
+    (128, 128, 1000, 3, 32, 31),    # 64 columns shared between tiles and one to align: past the pipelined kernels' window
+    (144, 200, 513, 2, 64, 33), (64, 96, 301, 3, 31, 1), (16, 16, 70, 2, 63, 62), (256, 128, 400, 5, 16, 30),
+    (64, 64, 1021, 3, 1, 1), (96, 96, 401, 5, 2, 4), (128, 128, 205, 5, 7, 14),  # ragged rows with few tiles: 9, 9, 12 pairs
+    (32, 64, 333, 3, 10, 10), (32, 32, 2047, 7, 1, 3),
+])
+def test_fallback_kernel(C_in, C_out, T, K, dil, pad):
+    """The kernel without a pipeline: windows of more than 128 columns, and ragged rows where it is the faster one; plain
+    and fused, with and without a residual, and the statistics that a pass over its output takes."""
+    say("conv fallback", C_in, C_out, T, K, dil, pad)
+    g = configs.rng(C_in + C_out + T + K + pad)
+    t = lambda a, dt=np.float32: torch.from_numpy(np.ascontiguousarray(a.astype(dt))).cuda()  # noqa: E731
+    B, T_out = 2, T + 2 * pad - dil * (K - 1)
+    x, w, b = t(g.standard_normal((B, C_in, T)) * 1.3 + 0.2), t(g.standard_normal((C_out, C_in, K)) * 0.05, np.float16), \
+        t(g.standard_normal(C_out), np.float16)
+    gam, bet, alp = t(g.standard_normal((B, C_in)) * 0.1), t(g.standard_normal((B, C_in)) * 0.1), t(g.uniform(0.5, 1.5, C_in))
+    r = t(g.standard_normal((B, C_out, T_out)))
+    wp = abi.conv1d_pack_f16(w)
+    d = x.double()
+    m = d.mean(-1, keepdim=True)
+    y = (d - m) / torch.sqrt((d - m).square().mean(-1, keepdim=True) + 1e-5)
+    y = y * (1.0 + gam.double()[:, :, None]) + bet.double()[:, :, None]
+    y = y + torch.sin(alp.double()[None, :, None] * y).square() / (alp.double()[None, :, None] + 1e-9)
+    for fused, src in ((False, d), (True, y)):
+        sp = torch.nn.functional.pad(src, (pad, pad))
+        ref = b.double()[None, :, None].expand(B, -1, T_out).clone()
+        mag = torch.zeros_like(ref)
+        for k in range(K):
+            for i in range(B):
+                s = sp[i, :, k * dil:k * dil + T_out].contiguous()
+                ref[i] += w[:, :, k].double().contiguous() @ s
+                mag[i] += w[:, :, k].double().abs().contiguous() @ s.abs()
+        for res in (None, r):
+            want = ref if res is None else ref + res.double()
+            bar = (2e-6 + C_in * K * 2.0 ** -24) * mag + 2.0 ** -22 * want.abs() + 2.0 ** -24 * r.double().abs() + 1e-30
+            for stats in (False, True):
+                buf = torch.full((B * C_out * T_out + 32,), -7.0, device="cuda")
+                out = buf[16:-16].view(B, C_out, T_out)
+                if fused:
+                    o, st = abi.adain_snake_conv1d_chain(x, gam, bet, alp, wp, b, res, want_stats=stats, padding=pad,
+                                                         dilation=dil, records=False, out=out)
+                elif stats:
+                    o, st = abi.conv1d_f16w_packed_stats(x, wp, b, res, padding=pad, dilation=dil, records=False, out=out)
+                else:
+                    o = abi.conv1d_f16w_packed(x, wp, b, res, padding=pad, dilation=dil, out=out)
+                assert bool((buf[:16] == -7.0).all()) and bool((buf[-16:] == -7.0).all()), "wrote outside the output"
+                worst = float(((o.double() - want).abs() / bar).max())
+                assert worst <= 1.0, f"fused={fused} residual={res is not None} stats={stats}: {worst:.2f} of the bar"
+                if stats:
+                    q = o.double().view(B * C_out, T_out)
+                    sd = torch.sqrt(q.var(-1, unbiased=False) + 1e-5)
+                    assert bool(((st[:, 0].double() - q.mean(-1)).abs() <= 2.0 ** -22 * (q.mean(-1).abs() + sd)).all())
+                    assert bool(((st[:, 1].double() * sd - 1.0).abs() <= 10 * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("C,T,K,dil", [(128, 16389, 3, 1), (128, 16388, 2, 5), (256, 1029, 3, 3), (256, 1028, 5, 1)])
+def test_one_launch_kernels_from_misaligned_views(C, T, K, dil):
+    """x, residual and output 4, 8 and 12 bytes past a 16-byte boundary on the resident-weight (C = 128) and the
+    streamed-weight kernel (C = 256): the results of aligned copies, bit for bit."""
+    say("conv one-launch misaligned", C, T, K, dil)
+    g = torch.Generator(device="cuda").manual_seed(C + T + K)
+    B, pad = 2, (K - 1) * dil // 2
+    T_out = T + 2 * pad - dil * (K - 1)
+    flat = lambda n: torch.randn(n + 8, generator=g, device="cuda")  # noqa: E731
+    xb, rb, ob = flat(B * C * T), flat(B * C * T_out), flat(B * C * T_out)
+    x, r, out = xb[1:1 + B * C * T].view(B, C, T), rb[2:2 + B * C * T_out].view(B, C, T_out), \
+        ob[3:3 + B * C * T_out].view(B, C, T_out)
+    wp = abi.conv1d_pack_f16((torch.randn((C, C, K), generator=g, device="cuda") * 0.05).half())
+    gam, bet = (torch.randn((B, C), generator=g, device="cuda") * 0.1 for _ in range(2))
+    alp = torch.rand(C, generator=g, device="cuda") + 0.5
+    kw = dict(padding=pad, dilation=dil, records=False)
+    want, ws = abi.adain_snake_conv1d_chain(x.clone(), gam, bet, alp, wp, None, r.clone(), **kw)
+    keep = ob.clone()
+    got, gs = abi.adain_snake_conv1d_chain(x, gam, bet, alp, wp, None, r, out=out, **kw)
+    assert torch.equal(got, want)
+    assert torch.equal(ob[:3], keep[:3]) and torch.equal(ob[3 + B * C * T_out:], keep[3 + B * C * T_out:])
+    assert bool(((gs - ws).abs() <= 2.0 ** -22 * ws.abs().clamp_min(1.0)).all())

@@ -6,12 +6,11 @@ products in the same order as the one-launch kernels (per output tile:
 input-channel chunks, then taps, then 16-channel steps, hi before lo), so
 each entry point's output must match its one-launch form bit for bit; the
 one-launch forms are checked against the oracle and float64 in
-test_gpu_conv1d.py and test_gpu_conv_chain.py. The record path is taken from
-K = 7 on; shapes: K = 7 / 8 / 9 / 11 at several dilations (an odd (K - 1)
-dilation among them), a partial 128-channel input chunk (C_in = 144, 96),
-two input chunks and two output blocks (C = 256, C_out = 200), batches,
-residuals, statistics handed along; and the one-launch fallbacks: K = 3 and
-5 (below the threshold), rows that are not 16-byte aligned, an odd C_out."""
+test_gpu_conv1d.py and test_gpu_conv_chain.py. Shapes: K = 7 / 8 / 9 / 11 at several dilations (an odd (K - 1)
+dilation among them), a partial 128-channel input chunk (C_in = 144, 96), two input chunks and two output blocks (C = 256,
+C_out = 200), K = 5 with several blocks, batches, residuals, statistics handed along; and calls without records either
+way: K = 3 and 5 with one channel block, an odd C_out. All of them fill less than a round of 128 x 128 tiles; the larger
+ones are in test_gpu_conv_record_tiles.py."""
 import numpy as np
 import pytest
 import torch
@@ -30,9 +29,9 @@ SHAPES = [  # B, C_in, C_out, T, K, dil, res
     (1, 96, 96, 3000, 9, 5, False),
     (3, 128, 64, 512, 11, 1, False),
     (2, 64, 96, 1001, 8, 1, False),   # (K - 1) dilation = 7, odd
-    (1, 128, 128, 4096, 3, 1, False),  # K < 7: the one-launch kernels both ways
+    (1, 128, 128, 4096, 3, 1, False),  # K < 7, one channel block: the one-launch kernels both ways
     (2, 144, 200, 1000, 5, 2, True),
-    (1, 64, 64, 601, 5, 2, False),    # T_out % 4 != 0: the one-launch kernels (no record path)
+    (1, 64, 64, 601, 5, 2, False),    # T % 4 != 0: the fallback kernel both ways
     (1, 128, 127, 1024, 7, 3, False),  # odd C_out: the one-launch kernels
 ]
 
@@ -69,9 +68,9 @@ def test_records_match_one_launch(B, C_in, C_out, T, K, dil, res):
     if T % 4 == 0:
         assert_bitexact(s1.cpu().numpy(), s0.cpu().numpy(), "adain_snake_conv1d_chain statistics")
     else:
-        # rows not 16-byte aligned on input: the one-launch path takes the statistics from a pass over its
-        # output instead of per-32-column partials, another summation order
-        assert_close(s1.cpu().numpy(), s0.cpu().numpy(), 1e-5, "adain_snake_conv1d_chain statistics")
+        # ragged rows: without records the fallback kernel may run, whose statistics are a pass over its output instead
+        # of per-32-column partials; each form is within 10 u of float64 (u = 2^-24, test_gpu_conv_ragged_rows.py)
+        assert_close(s1.cpu().numpy(), s0.cpu().numpy(), 20 * 2.0 ** -24, "adain_snake_conv1d_chain statistics")
     p1, q1 = abi.conv1d_f16w_packed_stats(x, wp, b, r, padding=pad, dilation=dil, records=True)
     p0 = abi.conv1d_f16w_packed(x, wp, b, r, padding=pad, dilation=dil)
     assert_bitexact(p1.cpu().numpy(), p0.cpu().numpy(), "conv1d_f16w_packed_stats vs conv1d_f16w_packed")
