@@ -37,7 +37,7 @@ typedef __attribute__((address_space(3))) nsr_float4 lds_f4;
 
 typedef _Float16 nsr_h8 __attribute__((ext_vector_type(8)));
 typedef float nsr_f32x16 __attribute__((ext_vector_type(16)));
-/* four f32 at any 4-byte aligned address (one 16-byte access) */
+/* Four f32 at any 4-byte aligned address (one 16-byte access). */
 typedef float cv_float4u __attribute__((ext_vector_type(4), aligned(4)));
 
 #define CV_TT 64            /* output columns per workgroup */
@@ -110,16 +110,16 @@ NSR_DEV cv_coef cv_row_coef(const nsr_conv_args& a, int b, int ci) {
 }
 
 
-/* Columns t .. t + 3 of an output row at byte offset `off`, `n` of them inside the row (n <= 0: none). A quad
+/* Columns t .. t + 3 of an output row at byte offset off + so (so wave-uniform), `n` of them inside the row (n <= 0: none). A quad
  * that the row's end cuts (rows with T_out % 4 != 0) is stored column by column; `ragged` (wave-uniform) says
  * that the tile may hold one. */
-NSR_DEV void store_quad(nsr_rsrc r, uint32_t off, nsr_float4 v, int n, bool ragged) {
-  if (n >= 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), r, off, 0, 0);
+NSR_DEV void store_quad(nsr_rsrc r, uint32_t off, nsr_float4 v, int n, bool ragged, uint32_t so = 0) {
+  if (n >= 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), r, off, so, 0);
   if (ragged) {
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
       const float ve = v[e]; /* a named copy: a bit_cast of the vector element itself reads element 0 */
-      if (n < 4 && e < n) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ve), r, off + 4u * e, 0, 0);
+      if (n < 4 && e < n) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ve), r, off + 4u * e, so, 0);
     }
   }
 }
@@ -1008,9 +1008,9 @@ NSR_CONV_PC(4)
  * on gfx950: the dwords of a 16-byte load or store inside the range are
  * served, the others read 0 or are dropped). The last quad of a row with
  * T_out % 4 != 0 is stored dword by dword, in the row's last column tile only.
- * At [4, 128, 57601], K = 11, the six stages of a ResBlock take 1429 us
- * against 2839 us on the kernel for unaligned rows above (MFMA kernel, records
- * and statistics together; 1394 us against 1319 us with T = 57600 on one box). */
+ * A ResBlock at [4, 128, 57601], K = 11 (six stages, records and statistics
+ * with them) takes 1412 us against 2842 us with such rows on the fallback
+ * kernel. */
 #define CV_RB 512           /* bytes per record */
 #define CV_RS 528           /* bytes per record slot in LDS */
 #define CV_RING 256         /* record slots in LDS */
@@ -1170,18 +1170,8 @@ NSR_DEV void conv_pr_body(const nsr_conv_args& a, const uint8_t* xs, const uint8
           if (p + 4 < 16) load_rq(p + 4);
         }
         /* C_out is even on this path: both rows of a pair exist or neither */
-        const uint32_t so = (uint32_t)(im.co0 + r0) * (uint32_t)a.T_out * 4u;
-        if (sok == 4u && im.co0 + r0 < a.C_out)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nsr_uint4, v), orr, svo, so, 0);
-        if (ragged && im.co0 + r0 < a.C_out) {
-          /* the quad that holds the row's end (T_out % 4 columns of it), last column tile only */
-#pragma unroll
-          for (int e = 0; e < 3; ++e) {
-            const float ve = v[e]; /* a named copy: a bit_cast of the vector element itself reads element 0 */
-            if (sok < 4u && (uint32_t)e < sok)
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ve), orr, svo + 4u * e, so, 0);
-          }
-        }
+        if (im.co0 + r0 < a.C_out)
+          store_quad(orr, svo, v, (int)sok, ragged, (uint32_t)(im.co0 + r0) * (uint32_t)a.T_out * 4u);
         for (int z = 0; z < gap; ++z) __builtin_amdgcn_s_sleep(1);
       }
     };
