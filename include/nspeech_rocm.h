@@ -196,10 +196,11 @@ nsr_status nsr_kv_cache_append(const void* new_kv, void* cache, nsr_dtype dtype,
  * elements between batches of gamma/beta (0 = shared over the batch, C =
  * per batch). alpha is per channel [C].
  * While a row fits on chip (x and out 16-byte aligned: T up to about 118,790;
- * other addresses: up to about 65k elements) x is read from HBM once and the statistics are
- * two passes over the on-chip row in f32 (the mean, then centred sums that
- * also correct the mean). Longer rows take a kernel that reads each row
- * twice (f64 sums, then the output; no scratch memory).
+ * other addresses: up to about 65k elements) x is read from HBM once and the
+ * statistics are one pass over the on-chip row in f32 (sum and sum of
+ * squares), with a second, centred pass when 4 mean^2 > var; rows of T % 4 != 0
+ * past 65,541 elements sum in f64. Longer rows take a kernel that reads each
+ * row twice (f64 sums, then the output; no scratch memory).
  * Replaces adain (src/kokoro/decoder.rs:1416-1428) followed by
  * snake_activation_tensor (:1471-1476), and
  * KokoroGpuBackend::adain_snake_f32 (src/kokoro/gpu_backend.rs:181-185,
@@ -406,10 +407,10 @@ nsr_status nsr_conv1d_f32io(const float* x, const void* w, const void* bias, flo
  *                          fragment order (ceil(C_out / 128) x 4 x K x
  *                          ceil(C_in / 128) x 8192 bytes). When the
  *                          workspace also covers it (after the parts the call
- *                          needs), rows of any length and alignment with
- *                          K >= 7 (K >= 3 when C_in or C_out is above 128),
- *                          even C_out and (K - 1) * dilation <= 56
- *                          take the two-launch record path: a
+ *                          needs), shapes with K >= 7 (K >= 3 when C_in or
+ *                          C_out is above 128), even C_out and
+ *                          (K - 1) * dilation <= 56 take the two-launch
+ *                          record path where it is the faster one: a
  *                          bandwidth-bound pass writes the records (AdaIN +
  *                          Snake included in the fused entry points) and the
  *                          fragment weights, then an MFMA kernel with no

@@ -9,16 +9,17 @@
  * gamma/beta come per (batch, channel) from the style Linear (precomputed and
  * rounded to f16 for the GPU backend, decoder.rs:966-981), alpha per channel.
  *
- * Row kernel (aligned rows: x, out 16-byte aligned, T % 4 == 0): the row is
- * read from HBM once into registers and LDS, its statistics are two passes
- * over the on-chip copy, and the output is written once: HBM traffic is the
- * algorithmic 8 bytes per element. Long rows run on a persistent grid that
- * overlaps the next row's reads with the current row's writes.
+ * Row kernel (x, out 16-byte aligned; a form of it for T % 4 != 0): the row is
+ * read from HBM once into registers and LDS, its statistics are one pass over
+ * the on-chip copy (a second, centred one when 4 mean^2 > var), and the output
+ * is written once: HBM traffic is the algorithmic 8 bytes per element. Long
+ * rows run on a persistent grid that overlaps the next row's reads with the
+ * current row's writes.
  *
- * Unaligned rows take the register-resident kernel further down (global
- * loads, partial edge chunks per element). Rows longer than the on-chip
- * budget take the long-row kernel at the end: f64 sum and sum of squares
- * over one read, then a second read to apply.
+ * Other rows take the register-resident kernel further down (global loads,
+ * partial edge chunks per element). Rows longer than the on-chip budget take
+ * the long-row kernel at the end: f64 sum and sum of squares over one read,
+ * then a second read to apply.
  */
 #include "device_common.h"
 
@@ -494,7 +495,7 @@ NSR_ADAIN_ROW(512, 39, 19)
 /* Rows that are not a multiple of 4 long, where the host's rule takes them (ragged_row_kernel). VGPR slots up to
  * 19, 19 LDS slots and an even number of VGPR slots beyond. What bounds it is what bounds the aligned rows; the chunks stay on the 16-byte grid, so no
  * access is split, and the edges cost one load and one store. Measured on MI355X, graph replays of one call, against
- * the kernels these rows took before (one workgroup per row; past T = 65,538 two reads of the row):
+ * the kernels these rows took before (one workgroup per row; past T = 65,541 two reads of the row):
  * [8, 128, 115201] 210 against 554 us ([8, 128, 115200] on the aligned kernel: 185), [1, 128, 115201] 31 against 130,
  * [4, 128, 57601] 51 against 53.5, [8, 128, 28801] 47.5 against 52.0. More than 32 slots sum in f64 (W): 0 to 1 us a
  * call, [1, 128, 115201] 29.9 against 29.4 us with f32 sums, [8, 128, 115201] 194 against 195 (inputs rotated). */
@@ -543,8 +544,8 @@ extern "C" __global__ void __launch_bounds__(512)
  * are partial and taken one element per lane by the last 8 lanes, the
  * interior chunks 1..nch-2 are full and spread as j = 1 + tid + BLOCK*k. Loads of the chunk
  * array are branch-free (index clamped in bounds, out-of-row slots zeroed by
- * a select), which keeps the array in VGPRs. Two-pass statistics over the
- * registers (mean, then centred sums with the corrected two-pass term). */
+ * a select), which keeps the array in VGPRs. Statistics as the row kernel's:
+ * one pass, a centred one when 4 mean^2 > var. */
 template <int BLOCK, int NV>
 NSR_DEV void adain_resident_u(const nsr_adain_args& a, int pdt) {
   NSR_NO_CONTRACT
